@@ -110,6 +110,23 @@ MKV_DEV void store_out8(void* out, int dt, int64_t off, const float* x) {
   }
 }
 
+// Store 4 consecutive fp32 values in the output dtype.
+MKV_DEV void store_out4(void* out, int dt, int64_t off, const float* x) {
+  if (dt == MKV_DTYPE_F32) {
+    *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(out) + off) = f32x4{x[0], x[1], x[2], x[3]};
+  } else {
+    u32x2 a;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const uint32_t lo = dt == MKV_DTYPE_BF16 ? f32_to_bf16_bits(x[2 * j]) : f32_to_f16_bits(x[2 * j]);
+      const uint32_t hi =
+          dt == MKV_DTYPE_BF16 ? f32_to_bf16_bits(x[2 * j + 1]) : f32_to_f16_bits(x[2 * j + 1]);
+      a[j] = lo | (hi << 16);
+    }
+    *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(out) + off) = a;
+  }
+}
+
 struct WorkItem {
   int b, kvh, split, num_splits;
   int t_begin, t_end;  // token range of this split (context lengths fit in 31 bits)
@@ -139,10 +156,19 @@ MKV_DEV int64_t wave_work_index() {
   return (int64_t)blockIdx.x * kDecWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 }
 
+// The output dims of a lane's accumulators acc[0..7][.]: 8c .. 8c+7 in the
+// 16-bit MFMA kernels; 4c .. 4c+3 and 64+4c .. 64+4c+3 in the fp32 kernels
+// (F32L), whose V loads take whole lines that way.  acc_dim = the dim of
+// acc[4 * half].
+template <bool F32L>
+MKV_DEV int acc_dim(int c, int half) {
+  return F32L ? 64 * half + 4 * c : 8 * c + 4 * half;
+}
+
 // Final normalisation / partial write for one wave.  Lane (kg, c) holds
-// O[head 4kg + r][dim 8c + mm] in acc[mm][r]; m_col / l_col hold the running
-// max and the (lane-group summed) denominator of head c.
-template <bool PAIR>
+// O[head 4kg + r][dims of acc_dim] in acc[mm][r]; m_col / l_col hold the
+// running max and the (lane-group summed) denominator of head c.
+template <bool PAIR, bool F32L>
 MKV_DEV void finish_item(const DecodeArgs& a, const WorkItem& it, f32x4 (&acc)[8], float m_col,
                          float l_col, float v_mul) {
   const int lane = threadIdx.x & 63;
@@ -159,20 +185,26 @@ MKV_DEV void finish_item(const DecodeArgs& a, const WorkItem& it, f32x4 (&acc)[8
       const float inv = lh > 0.0f ? v_mul / lh : 0.0f;
 #pragma unroll
       for (int mm = 0; mm < 8; ++mm) x[mm] = acc[mm][r] * inv;
-      int col0;
-      if (out_cols<PAIR>(a.group, h, c, col0))
-        store_out8(a.out, a.q_dtype, (int64_t)it.b * a.out_stride + (int64_t)hq * kQDim<PAIR> + col0, x);
+      const int64_t row = (int64_t)it.b * a.out_stride + (int64_t)hq * kQDim<PAIR>;
+      if constexpr (F32L) {
+        const bool hi = PAIR && h >= (a.group >> 1);  // a paired head stores its own half
+        if (!PAIR || !hi) store_out4(a.out, a.q_dtype, row + 4 * c, x);
+        if (!PAIR || hi) store_out4(a.out, a.q_dtype, row + 4 * c + (PAIR ? 0 : 64), x + 4);
+      } else {
+        int col0;
+        if (out_cols<PAIR>(a.group, h, c, col0)) store_out8(a.out, a.q_dtype, row + col0, x);
+      }
     } else {
       const int64_t slot = ((int64_t)it.b * a.num_heads + hq) * a.max_splits + it.split;
-      float* p = a.ws_acc + slot * kHeadDim + 8 * c;
+      float* p = a.ws_acc + slot * kHeadDim;
       u32x4 lo, hi;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         lo[j] = __float_as_uint(acc[j][r]);
         hi[j] = __float_as_uint(acc[4 + j][r]);
       }
-      st16(p, lo);
-      st16(p + 4, hi);
+      st16(p + acc_dim<F32L>(c, 0), lo);
+      st16(p + acc_dim<F32L>(c, 1), hi);
       if (c == 0) {
         a.ws_ml[slot * 2] = mh;
         a.ws_ml[slot * 2 + 1] = lh;
@@ -764,7 +796,7 @@ MKV_DEV void split_decode(const DecodeArgs& a) {
   float l_col = l_run + __shfl_xor(l_run, 16);
   l_col += __shfl_xor(l_col, 32);
   const float v_mul = (KV_DT == MKV_DTYPE_FP8E4M3) ? load_uniform_f32(a.v_scale) : 1.0f;
-  finish_item<PAIR>(a, it, acc, m_run, l_col, v_mul);
+  finish_item<PAIR, false>(a, it, acc, m_run, l_col, v_mul);
 }
 
 template <int KV_DT, bool PAIR>
@@ -792,36 +824,17 @@ paged_decode_mfma16_2w_kernel(DecodeArgs a) {
 // ---------------------------------------------------------------------------
 constexpr int kWgMaxWaves = 8;
 
-// The LDS merge of the workgroup route: every wave writes its (acc, m, l)
-// (lane (kg, c) holds O[head 4kg + r][dim 8c + mm] in acc[mm][r], m and l of
-// head c), then the workgroup combines the nw partials of each (head, 8-dim
-// chunk) with the log-sum-exp rule and writes the output row.  v_mul: the
-// per-tensor V scale (1 otherwise).
+// The workgroup's merge once every wave has written its (acc, m, l) to LDS:
+// the nw partials of each (head, 8-dim chunk) combined with the log-sum-exp
+// rule, one output row a head.  v_mul: the per-tensor V scale (1 otherwise).
 template <bool PAIR>
-MKV_DEV void wg_merge_store(const DecodeArgs& a, const WorkItem& it, const f32x4 (&acc)[8], float m_run,
-                            float l_col, float v_mul) {
+MKV_DEV void wg_merge_combine(const DecodeArgs& a, const WorkItem& it, float v_mul) {
   extern __shared__ float wg_lds[];
   const int nw = blockDim.x >> 6;
-  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  const int c = lane & 15, kg = lane >> 4;
   const int G = a.group;
   float* acc_l = wg_lds;
   float* m_l = wg_lds + nw * G * kHeadDim;
   float* l_l = m_l + nw * G;
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int h = 4 * kg + r;
-    if (h < G) {
-      float* p = acc_l + (wv * G + h) * kHeadDim + 8 * c;
-      *reinterpret_cast<f32x4*>(p) = f32x4{acc[0][r], acc[1][r], acc[2][r], acc[3][r]};
-      *reinterpret_cast<f32x4*>(p + 4) = f32x4{acc[4][r], acc[5][r], acc[6][r], acc[7][r]};
-    }
-  }
-  if (kg == 0 && c < G) {
-    m_l[wv * G + c] = m_run;
-    l_l[wv * G + c] = l_col;
-  }
   __syncthreads();
   for (int u = threadIdx.x; u < G * 16; u += blockDim.x) {
     const int h = u >> 4, d0 = (u & 15) * 8;
@@ -852,6 +865,36 @@ MKV_DEV void wg_merge_store(const DecodeArgs& a, const WorkItem& it, const f32x4
   }
 }
 
+// The LDS merge of the workgroup route: every wave writes its (acc, m, l)
+// (lane (kg, c) holds O[head 4kg + r][dims of acc_dim] in acc[mm][r], m and l
+// of head c), then the workgroup combines them.
+template <bool PAIR, bool F32L = false>
+MKV_DEV void wg_merge_store(const DecodeArgs& a, const WorkItem& it, const f32x4 (&acc)[8], float m_run,
+                            float l_col, float v_mul) {
+  extern __shared__ float wg_lds[];
+  const int nw = blockDim.x >> 6;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int c = lane & 15, kg = lane >> 4;
+  const int G = a.group;
+  float* acc_l = wg_lds;
+  float* m_l = wg_lds + nw * G * kHeadDim;
+  float* l_l = m_l + nw * G;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int h = 4 * kg + r;
+    if (h < G) {
+      float* p = acc_l + (wv * G + h) * kHeadDim;
+      *reinterpret_cast<f32x4*>(p + acc_dim<F32L>(c, 0)) = f32x4{acc[0][r], acc[1][r], acc[2][r], acc[3][r]};
+      *reinterpret_cast<f32x4*>(p + acc_dim<F32L>(c, 1)) = f32x4{acc[4][r], acc[5][r], acc[6][r], acc[7][r]};
+    }
+  }
+  if (kg == 0 && c < G) {
+    m_l[wv * G + c] = m_run;
+    l_l[wv * G + c] = l_col;
+  }
+  wg_merge_combine<PAIR>(a, it, v_mul);
+}
 // Work item of wave wv of the workgroup route: the sequence's 32-token tiles
 // cut into nw consecutive ranges.
 MKV_DEV WorkItem wg_item(const DecodeArgs& a) {
@@ -1415,13 +1458,52 @@ paged_decode_wg_produce_kernel(ProduceDecodeArgs f) {
 // fp32 caches on the workgroup route: 16-token tiles on v_mfma_f32_16x16x4_f32
 // (the split-K fp32 kernel's arithmetic), loaded through per-tile buffer
 // descriptors one tile ahead of the math.
+//
+// Every load instruction covers whole 128-byte lines: a 512-byte K row is
+// four lines, and line p of the 16 rows is read by two instructions of eight
+// lanes a row and one exchange (fp8_k_lanes, k_exchange: an FP8 row is one
+// such line), which leaves lane (c, kg) with dims 32p + 8kg .. +7 of row c
+// (the contraction order is free); a V instruction reads 256 consecutive
+// bytes of four rows, so a lane's output dims are 4c .. +3 and 64+4c .. +3.
+// Read as 128 consecutive bytes a lane, each K instruction touched 64 lines
+// for 16 bytes of each, and the eight that share those lines did not find
+// them in the L1 again.
+// SMALL (at most four query heads per KV head; with head pairing four per
+// cache head): the K rows lie where v_mfma_f32_4x4x1_16b_f32 wants them, row
+// 4kg + (c & 3) and dims 32p + 8 (c >> 2) .. +7 on lane (c, kg), and the
+// exchange is between neighbouring lanes.
 struct TileF32 {
-  u32x4 k[8];     // K row of token t0 + c, dims 32kg .. 32kg+31
-  u32x4 v[4][2];  // V rows of tokens t0 + 4kg + r, dims 8c .. 8c+7
+  u32x4 k[8];     // piece i of line p in k[2p + i], before the exchange
+  u32x4 v[4][2];  // V rows of tokens t0 + 4kg + r, dims 4c and 64 + 4c
   bool ok;        // block present
 };
 
+// fp8_k_lanes and k_exchange for SMALL: even lanes read their own row in
+// instruction A and their odd neighbour's in B, odd lanes the other way round.
+MKV_DEV Fp8KLanes f32_small_k_lanes(int row_bytes) {
+  const int lane = threadIdx.x & 63;
+  const int odd = lane & 1, chunk = (lane >> 2) & 3;
+  Fp8KLanes f;
+  f.row_a = 4 * (lane >> 4) + (lane & 2);
+  f.row_b = f.row_a + 1;
+  f.off_a = f.row_a * row_bytes + 32 * chunk + (odd ? 16 : 0);
+  f.off_b = f.row_b * row_bytes + 32 * chunk + (odd ? 0 : 16);
+  return f;
+}
+MKV_DEV void k_exchange_pairs(u32x4& a, u32x4& b) {
+  const bool odd = threadIdx.x & 1;
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    const uint32_t send = odd ? a[d] : b[d];
+    const uint32_t own = odd ? b[d] : a[d];
+    // quad_perm [1, 0, 3, 2]: from the neighbouring lane
+    b[d] = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)send, 0xb1, 0xf, 0xf, false);
+    a[d] = own;
+  }
+}
+
 // The loads of the 16-token tile at t0 in block phys (item_phys1).
+template <bool SMALL>
 MKV_DEV void load_tile_f32(const DecodeArgs& a, const WorkItem& it, const ItemLoad& L, int t0, int64_t phys,
                            TileF32& T) {
   const int lane = threadIdx.x & 63;
@@ -1431,14 +1513,20 @@ MKV_DEV void load_tile_f32(const DecodeArgs& a, const WorkItem& it, const ItemLo
   const __amdgpu_buffer_rsrc_t rk = rows_rsrc(a.k_cache, phys, L.blk_bytes, off);
   const __amdgpu_buffer_rsrc_t rv = rows_rsrc(a.v_cache, phys, L.blk_bytes, off);
   T.ok = phys >= 0;
-  const uint32_t ko = (t0 + c < it.t_end) ? (uint32_t)L.k_voff : kOob;
+  const Fp8KLanes kl = SMALL ? f32_small_k_lanes(L.row_bytes) : fp8_k_lanes(L.row_bytes);
+  const uint32_t ka = t0 + kl.row_a < it.t_end ? (uint32_t)kl.off_a : kOob;
+  const uint32_t kb = t0 + kl.row_b < it.t_end ? (uint32_t)kl.off_b : kOob;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) T.k[i] = __builtin_amdgcn_raw_buffer_load_b128(rk, ko + 16 * i, 0, kAuxNt);
+  for (int p = 0; p < 4; ++p) {
+    T.k[2 * p] = __builtin_amdgcn_raw_buffer_load_b128(rk, ka + 128 * p, 0, kAuxNt);
+    T.k[2 * p + 1] = __builtin_amdgcn_raw_buffer_load_b128(rk, kb + 128 * p, 0, kAuxNt);
+  }
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    const uint32_t vo = (t0 + 4 * kg + r < it.t_end) ? (uint32_t)(L.v_voff + r * L.row_bytes) : kOob;
+    const uint32_t vo =
+        (t0 + 4 * kg + r < it.t_end) ? (uint32_t)((4 * kg + r) * L.row_bytes + 16 * c) : kOob;
     T.v[r][0] = __builtin_amdgcn_raw_buffer_load_b128(rv, vo, 0, kAuxNt);
-    T.v[r][1] = __builtin_amdgcn_raw_buffer_load_b128(rv, vo + 16, 0, kAuxNt);
+    T.v[r][1] = __builtin_amdgcn_raw_buffer_load_b128(rv, vo + 256, 0, kAuxNt);
   }
 }
 
@@ -1447,8 +1535,16 @@ MKV_DEV void compute_tile_f32(const TileF32& T, int t0, int t_end, const float (
   const int kg = (threadIdx.x & 63) >> 4;
   f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int st = 0; st < 32; ++st)
-    s = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(T.k[st >> 2][st & 3]), qf[st], s, 0, 0, 0);
+  for (int p = 0; p < 4; ++p) {
+    u32x4 k0 = T.k[2 * p], k1 = T.k[2 * p + 1];
+    k_exchange(k0, k1);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      s = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(k0[j]), qf[8 * p + j], s, 0, 0, 0);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      s = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(k1[j]), qf[8 * p + 4 + j], s, 0, 0, 0);
+  }
   float mx = kNegBig;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
@@ -1485,61 +1581,277 @@ MKV_DEV void compute_tile_f32(const TileF32& T, int t0, int t_end, const float (
   }
 }
 
+// Running state of one wave.  Not SMALL: acc[mm][r] holds O[head 4kg + r], m
+// and l[0] belong to head c.  SMALL: acc[mm][r] holds head r's sum over the
+// tokens of this lane's kg (added over kg at the end), m and l[0] belong to
+// head c & 3; with head pairing acc[0..3] and m / l[0] are those of the cache
+// head 2v's query heads, acc[4..7] and m / l[1] of 2v + 1's.
+template <bool PAIR, bool SMALL>
+struct F32State {
+  static constexpr int kSets = PAIR && SMALL ? 2 : 1;
+  f32x4 acc[8];
+  float m[kSets], l[kSets];
+  MKV_DEV F32State() {
+#pragma unroll
+    for (int mm = 0; mm < 8; ++mm) acc[mm] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < kSets; ++i) {
+      m[i] = kNegBig;
+      l[i] = 0.0f;
+    }
+  }
+};
+
+// Value of lane N of this lane's group of four (quad_perm).
+template <int N>
+MKV_DEV float quad_bcast(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x55 * N, 0xf, 0xf, true));
+}
+
+// A tile for at most four query heads on v_mfma_f32_4x4x1_16b_f32: sixteen
+// independent 4x4 products an instruction, at the same rate of products as
+// 16x16x4 but with none of its columns idle beyond the fourth (for two query
+// heads, 512 matrix cycles a tile in place of 2048, which bound the
+// 16x16x4 form: a CU's 8 waves took 1.7 us a tile).  QK: block (kg, c >> 2)
+// multiplies tokens 4kg .. +3 and a quarter of the dims, one per
+// instruction; the four quarters are added with two row rotates, and lane
+// (c, kg) holds the scores of head c & 3 and those tokens.  PV: block (kg,
+// c >> 2) takes P from the lane that holds it and the four lanes' V dims.
+template <bool PAIR>
+MKV_DEV void compute_tile_f32_small(const TileF32& T, int t0, int t_end, const float (&qf)[32],
+                                    float score_mul, F32State<PAIR, true>& st) {
+  constexpr int kSets = F32State<PAIR, true>::kSets;
+  const int kg = (threadIdx.x & 63) >> 4;
+  f32x4 s[kSets][2];
+#pragma unroll
+  for (int i = 0; i < kSets; ++i) s[i][0] = s[i][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int p = 0; p < 4; ++p) {
+    u32x4 k0 = T.k[2 * p], k1 = T.k[2 * p + 1];
+    k_exchange_pairs(k0, k1);
+    f32x4(&sp)[2] = s[PAIR ? p >> 1 : 0];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      sp[0] = __builtin_amdgcn_mfma_f32_4x4x1f32(__uint_as_float(k0[j]), qf[8 * p + j], sp[0], 0, 0, 0);
+      sp[1] = __builtin_amdgcn_mfma_f32_4x4x1f32(__uint_as_float(k1[j]), qf[8 * p + 4 + j], sp[1], 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < kSets; ++i) {
+    float sc[4], mx = kNegBig;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      float x = s[i][0][r] + s[i][1][r];
+      x += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x128, 0xf, 0xf, true));  // row_ror:8
+      x += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x124, 0xf, 0xf, true));  // row_ror:4
+      const bool ok = t0 + 4 * kg + r < t_end && T.ok;
+      sc[r] = ok ? x * score_mul : -__builtin_huge_valf();
+      mx = fmaxf(mx, sc[r]);
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 16));
+    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    const float m_new = fmaxf(st.m[i], mx);
+    const float alpha = __builtin_amdgcn_exp2f(st.m[i] - m_new);
+    st.m[i] = m_new;
+    float psum = 0.0f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      sc[r] = __builtin_amdgcn_exp2f(sc[r] - m_new);
+      psum += sc[r];
+    }
+    st.l[i] = st.l[i] * alpha + psum;
+    const int m0 = PAIR ? 4 * i : 0, m1 = PAIR ? 4 * i + 4 : 8;
+    if (__builtin_amdgcn_ballot_w64(alpha != 1.0f)) {
+      const f32x4 ar = {quad_bcast<0>(alpha), quad_bcast<1>(alpha), quad_bcast<2>(alpha), quad_bcast<3>(alpha)};
+#pragma unroll
+      for (int mm = m0; mm < m1; ++mm) st.acc[mm] *= ar;
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int mm = m0; mm < m1; ++mm)
+        st.acc[mm] = __builtin_amdgcn_mfma_f32_4x4x1f32(sc[r], __uint_as_float(T.v[r][mm >> 2][mm & 3]),
+                                                        st.acc[mm], 0, 0, 0);
+  }
+}
+
+// The end of a wave's range: sums over the lane groups, so that lanes of kg 0
+// hold whole sums (SMALL), or lane c of every kg l of head c.
+template <bool PAIR, bool SMALL>
+MKV_DEV void f32_close(F32State<PAIR, SMALL>& st) {
+#pragma unroll
+  for (int i = 0; i < F32State<PAIR, SMALL>::kSets; ++i) {
+    st.l[i] += __shfl_xor(st.l[i], 16);
+    st.l[i] += __shfl_xor(st.l[i], 32);
+  }
+  if constexpr (SMALL) {
+#pragma unroll
+    for (int mm = 0; mm < 8; ++mm)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        st.acc[mm][r] += __shfl_xor(st.acc[mm][r], 16);
+        st.acc[mm][r] += __shfl_xor(st.acc[mm][r], 32);
+      }
+  }
+}
+
+// SMALL: query head of acc[4 half ..][r] and of m / l, or -1 past the group.
+template <bool PAIR>
+MKV_DEV int f32_small_head(const DecodeArgs& a, int half, int r) {
+  const int g = PAIR ? a.group >> 1 : a.group;
+  return r < g ? r + (PAIR ? half * g : 0) : -1;
+}
+
+// SMALL: wg_merge_store and finish_item for f32_close's sums.
+template <bool PAIR>
+MKV_DEV void wg_merge_store_f32_small(const DecodeArgs& a, const WorkItem& it, const F32State<PAIR, true>& st) {
+  extern __shared__ float wg_lds[];
+  const int nw = blockDim.x >> 6;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int G = a.group;
+  float* m_l = wg_lds + nw * G * kHeadDim;
+  float* l_l = m_l + nw * G;
+  if (lane < 16) {
+#pragma unroll
+    for (int half = 0; half < 2; ++half)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int h = f32_small_head<PAIR>(a, half, r);
+        if (h >= 0)
+          *reinterpret_cast<f32x4*>(wg_lds + (wv * G + h) * kHeadDim + acc_dim<true>(lane, half)) =
+              f32x4{st.acc[4 * half][r], st.acc[4 * half + 1][r], st.acc[4 * half + 2][r], st.acc[4 * half + 3][r]};
+      }
+  }
+  if (lane < 4) {
+#pragma unroll
+    for (int i = 0; i < F32State<PAIR, true>::kSets; ++i) {
+      const int h = f32_small_head<PAIR>(a, i, lane);
+      if (h >= 0) {
+        m_l[wv * G + h] = st.m[i];
+        l_l[wv * G + h] = st.l[i];
+      }
+    }
+  }
+  wg_merge_combine<PAIR>(a, it, 1.0f);
+}
+
+template <bool PAIR>
+MKV_DEV void finish_item_f32_small(const DecodeArgs& a, const WorkItem& it, const F32State<PAIR, true>& st) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int half = 0; half < 2; ++half)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int h = f32_small_head<PAIR>(a, half, r);
+      const float lh = __shfl(st.l[PAIR ? half : 0], r);
+      const float mh = __shfl(st.m[PAIR ? half : 0], r);
+      if (h < 0 || lane >= 16) continue;
+      const int hq = it.kvh * a.group + h;
+      float x[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[j] = st.acc[4 * half + j][r];
+      if (it.num_splits == 1) {
+        const float inv = lh > 0.0f ? 1.0f / lh : 0.0f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) x[j] *= inv;
+        store_out4(a.out, a.q_dtype,
+                   (int64_t)it.b * a.out_stride + (int64_t)hq * kQDim<PAIR> + 4 * lane + (PAIR ? 0 : 64 * half), x);
+      } else {
+        const int64_t slot = ((int64_t)it.b * a.num_heads + hq) * a.max_splits + it.split;
+        *reinterpret_cast<f32x4*>(a.ws_acc + slot * kHeadDim + acc_dim<true>(lane, half)) =
+            f32x4{x[0], x[1], x[2], x[3]};
+        if (lane == 0 && (PAIR || half == 0)) {
+          a.ws_ml[slot * 2] = mh;
+          a.ws_ml[slot * 2 + 1] = lh;
+        }
+      }
+    }
+}
+
 // The fp32 tile pipeline of one wave over its range [t_begin, t_end): the
 // loads of tile i+1 in flight while tile i is computed, the block-table entry
 // of tile i+2 (a scalar load) while tile i+1's loads go out.
+template <bool PAIR, bool SMALL>
 MKV_DEV void f32_range(const DecodeArgs& a, const WorkItem& it, const float (&qf)[32], float score_mul,
-                       f32x4 (&acc)[8], float& m_run, float& l_run) {
+                       F32State<PAIR, SMALL>& st) {
   if (it.t_begin >= it.t_end) return;
+  auto compute = [&](const TileF32& T, int t0) {
+    if constexpr (SMALL)
+      compute_tile_f32_small<PAIR>(T, t0, it.t_end, qf, score_mul, st);
+    else
+      compute_tile_f32(T, t0, it.t_end, qf, score_mul, st.acc, st.m[0], st.l[0]);
+  };
   const ItemLoad Ld = item_load_setup<MKV_DTYPE_F32>(a, it);
   TileF32 ta, tb;
-  load_tile_f32(a, it, Ld, it.t_begin, item_phys1(a, it.b, it.t_begin, it.t_end), ta);
+  load_tile_f32<SMALL>(a, it, Ld, it.t_begin, item_phys1(a, it.b, it.t_begin, it.t_end), ta);
   int64_t ph = item_phys1(a, it.b, it.t_begin + 16, it.t_end);
   for (int t0 = it.t_begin;;) {
-    load_tile_f32(a, it, Ld, t0 + 16, ph, tb);
+    load_tile_f32<SMALL>(a, it, Ld, t0 + 16, ph, tb);
     ph = item_phys1(a, it.b, t0 + 32, it.t_end);
-    compute_tile_f32(ta, t0, it.t_end, qf, score_mul, acc, m_run, l_run);
+    compute(ta, t0);
     t0 += 16;
     if (t0 >= it.t_end) break;
-    load_tile_f32(a, it, Ld, t0 + 16, ph, ta);
+    load_tile_f32<SMALL>(a, it, Ld, t0 + 16, ph, ta);
     ph = item_phys1(a, it.b, t0 + 32, it.t_end);
-    compute_tile_f32(tb, t0, it.t_end, qf, score_mul, acc, m_run, l_run);
+    compute(tb, t0);
     t0 += 16;
     if (t0 >= it.t_end) break;
   }
 }
 
-// q of item (b, kvh) as fp32 for the fp32 kernels (same lane slice as the
-// 16-bit kernels).
-template <bool PAIR>
+// q of item (b, kvh) as fp32 for the fp32 kernels: lane (c, kg) holds dims
+// 32p + 8kg .. +7 of head c, p = 0..3 (TileF32's K dims), zeros for a padding
+// head and for the other half of a paired head; SMALL: dims 32p + 8 (c >> 2)
+// .. +7 of head c & 3 (with head pairing of the cache head whose line p is).
+template <bool PAIR, bool SMALL>
 MKV_DEV void load_q_f32(const DecodeArgs& a, int b, int kvh, float (&qf)[32]) {
   const int lane = threadIdx.x & 63;
-  const int c = lane & 15, kg = lane >> 4;
-  int d0;
-  if (q_slice<PAIR>(a.group, c, kg, d0)) {
-    const int64_t qoff = (int64_t)b * a.q_stride + (int64_t)(kvh * a.group + c) * kQDim<PAIR> + d0;
-    load_q32(a.q, a.q_dtype, qoff, qf);
-  } else {
+  const int c = lane & 15, kg = SMALL ? c >> 2 : lane >> 4;
 #pragma unroll
-    for (int i = 0; i < 32; ++i) qf[i] = 0.0f;
+  for (int p = 0; p < 4; ++p) {
+    const int h = SMALL ? f32_small_head<PAIR>(a, p >> 1, c & 3) : (c < a.group ? c : -1);
+    const bool hi = PAIR && h >= (a.group >> 1);
+    if (h >= 0 && (!PAIR || (p >= 2) == hi)) {
+      const int64_t off = (int64_t)b * a.q_stride + (int64_t)(kvh * a.group + h) * kQDim<PAIR> + 8 * kg +
+                          32 * (PAIR ? p & 1 : p);
+      if (a.q_dtype == MKV_DTYPE_F32) {
+        const float* q = reinterpret_cast<const float*>(a.q) + off;
+        const u32x4 x0 = ld16(q), x1 = ld16(q + 4);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          qf[8 * p + j] = __uint_as_float(x0[j]);
+          qf[8 * p + 4 + j] = __uint_as_float(x1[j]);
+        }
+      } else {
+        const u32x4 x = ld16(reinterpret_cast<const uint16_t*>(a.q) + off);
+        const bool bf = a.q_dtype == MKV_DTYPE_BF16;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          qf[8 * p + 2 * j] = bf ? bf16_bits_to_f32(x[j] & 0xffffu) : f16_bits_to_f32(x[j] & 0xffffu);
+          qf[8 * p + 2 * j + 1] = bf ? bf16_bits_to_f32(x[j] >> 16) : f16_bits_to_f32(x[j] >> 16);
+        }
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) qf[8 * p + j] = 0.0f;
+    }
   }
 }
 
-template <bool PAIR>
+template <bool PAIR, bool SMALL>
 __global__ __launch_bounds__(kWgMaxWaves* kWave) __attribute__((amdgpu_waves_per_eu(2))) void
 paged_decode_wg_f32_kernel(DecodeArgs a) {
   const WorkItem it = wg_item(a);
   float qf[32];
-  load_q_f32<PAIR>(a, it.b, it.kvh, qf);
-  const float score_mul = a.sm_scale * kLog2e;
-  f32x4 acc[8];
-#pragma unroll
-  for (int mm = 0; mm < 8; ++mm) acc[mm] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m_run = kNegBig, l_run = 0.0f;
-  f32_range(a, it, qf, score_mul, acc, m_run, l_run);
-  float l_col = l_run + __shfl_xor(l_run, 16);
-  l_col += __shfl_xor(l_col, 32);
-  wg_merge_store<PAIR>(a, it, acc, m_run, l_col, 1.0f);
+  load_q_f32<PAIR, SMALL>(a, it.b, it.kvh, qf);
+  F32State<PAIR, SMALL> st;
+  f32_range<PAIR, SMALL>(a, it, qf, a.sm_scale * kLog2e, st);
+  f32_close<PAIR, SMALL>(st);
+  if constexpr (SMALL)
+    wg_merge_store_f32_small<PAIR>(a, it, st);
+  else
+    wg_merge_store<PAIR, true>(a, it, st.acc, st.m[0], st.l[0], 1.0f);
 }
 
 // ---------------------------------------------------------------------------
@@ -2243,13 +2555,81 @@ MKV_DEV void store_out2(const DecodeArgs& a, int64_t off, float x0, float x1) {
 // Merge of stream-K partials: one wave per (sequence, query head).  The
 // partials of an item (sequence, KV head kvh) come from wave kvh of the
 // consecutive groups glo..ghi, one slot each.
-// Lane i reads (m, l) of contributor wlo + i, so the maximum and the
-// denominator are wave reductions rather than a chain of dependent loads, and
-// the accumulator rows are read four contributors at a time (independent
-// loads in flight) with each contributor's weight taken from its lane.
 MKV_DEV int merge_slot(const DecodeArgs& a, int glo, int s0, int grp, int kvh, int h) {
   const int wp = grp * a.num_kv_heads + sk_slot(kvh, a.num_kv_heads);
   return ((wp * 2 + (grp == glo ? s0 : 0)) * a.group + h);
+}
+
+// Log-sum-exp combination of nc >= 1 partials of one query head, slots
+// base + slot(0 .. nc-1) of the workspace: the lane's two dims in o0 / o1 and
+// the denominator (reduced over the wave) in l.  Lane i reads (m, l) of
+// partial c0 + i, so the maximum and the denominator are wave reductions; up
+// to 64 partials take one round trip for every (m, l) and the first four
+// accumulator rows (their slots do not depend on (m, l)), then one for every
+// eight rows more.
+template <typename Slot>
+MKV_DEV void merge_partials(const DecodeArgs& a, int64_t base, int nc, Slot slot, float& o0, float& o1,
+                            float& l) {
+  const int lane = threadIdx.x & 63;
+  const float* acc = a.ws_acc + base * kHeadDim + 2 * lane;
+  const float* mls = a.ws_ml + base * 2;
+  o0 = o1 = l = 0.0f;
+  auto row = [&](int sl) { return *reinterpret_cast<const f32x2*>(acc + (int64_t)sl * kHeadDim); };
+  auto weight = [&](float wgt, int j) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wgt), j)); };
+  // rows j0 .. of the partials held by the lanes (cnt of them), eight at a
+  // time; past the last one row 0 is read again and weighs nothing
+  auto rest = [&](int my_slot, float wgt, int j0, int cnt) {
+    for (int j = j0; j < cnt; j += 8) {
+      f32x2 y[8];
+      float w8[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const bool in = j + u < cnt;
+        y[u] = row(__builtin_amdgcn_readlane(my_slot, in ? j + u : 0));
+        w8[u] = in ? weight(wgt, j + u) : 0.0f;
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        o0 += w8[u] * y[u][0];
+        o1 += w8[u] * y[u][1];
+      }
+    }
+  };
+  if (nc <= kWave) {
+    const int my_slot = lane < nc ? slot(lane) : 0;
+    f32x2 x[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) x[u] = row(__builtin_amdgcn_readlane(my_slot, u < nc ? u : 0));
+    const f32x2 ml = lane < nc ? *reinterpret_cast<const f32x2*>(mls + (int64_t)my_slot * 2)
+                               : f32x2{kNegBig, 0.0f};
+    const float M = wave_max(ml[0]);
+    const float wgt = lane < nc ? __builtin_amdgcn_exp2f(ml[0] - M) : 0.0f;
+    l = wgt * ml[1];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {  // lanes past the last partial weigh nothing
+      const float w1 = weight(wgt, u);
+      o0 += w1 * x[u][0];
+      o1 += w1 * x[u][1];
+    }
+    rest(my_slot, wgt, 4, nc);
+  } else {
+    float M = kNegBig;
+    for (int c0 = 0; c0 < nc; c0 += kWave)
+      if (c0 + lane < nc) M = fmaxf(M, mls[(int64_t)slot(c0 + lane) * 2]);
+    M = wave_max(M);
+    for (int c0 = 0; c0 < nc; c0 += kWave) {
+      int my_slot = 0;
+      float wgt = 0.0f;
+      if (c0 + lane < nc) {
+        my_slot = slot(c0 + lane);
+        wgt = __builtin_amdgcn_exp2f(mls[(int64_t)my_slot * 2] - M);
+        l += wgt * mls[(int64_t)my_slot * 2 + 1];
+      }
+      rest(my_slot, wgt, 0, nc - c0 < kWave ? nc - c0 : kWave);
+    }
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) l += __shfl_xor(l, o);
 }
 
 __global__ __launch_bounds__(kDecWaves* kWave) void paged_decode_stream_merge_kernel(DecodeArgs a,
@@ -2268,87 +2648,7 @@ __global__ __launch_bounds__(kDecWaves* kWave) void paged_decode_stream_merge_ke
   if (n > 0) {
     const int glo = meta[0], ghi = meta[1], s0 = meta[2];
     if (glo == ghi) return;  // written whole by the main kernel
-    const int nc = ghi - glo + 1;
-    if (nc <= kWave) {
-      // One round trip for the common case: every contributor's (m, l),
-      // lane-parallel, and the first four accumulator rows are loaded
-      // together (the rows' slots do not depend on (m, l)); the weights
-      // follow from the maximum, the remaining rows four at a time.
-      const int my_slot = lane < nc ? merge_slot(a, glo, s0, glo + lane, kvh, h) : 0;
-      f32x2 x[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {  // nc >= 2; rows u >= nc repeat row 0 with weight 0
-        const int64_t sl = __builtin_amdgcn_readlane(my_slot, u);
-        x[u] = *reinterpret_cast<const f32x2*>(a.ws_acc + (u < nc ? sl : 0) * kHeadDim + 2 * lane);
-      }
-      const f32x2 ml = lane < nc ? *reinterpret_cast<const f32x2*>(a.ws_ml + (int64_t)my_slot * 2)
-                                 : f32x2{kNegBig, 0.0f};
-      const float M = wave_max(ml[0]);
-      const float wgt = lane < nc ? __builtin_amdgcn_exp2f(ml[0] - M) : 0.0f;
-      l = wgt * ml[1];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const float w1 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wgt), u));
-        o0 += w1 * x[u][0];
-        o1 += w1 * x[u][1];
-      }
-      for (int j = 4; j < nc; j += 4) {
-        f32x2 y[4];
-        float w4[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int64_t sl = __builtin_amdgcn_readlane(my_slot, j + u < nc ? j + u : 0);
-          w4[u] = j + u < nc ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wgt), j + u)) : 0.0f;
-          y[u] = *reinterpret_cast<const f32x2*>(a.ws_acc + sl * kHeadDim + 2 * lane);
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          o0 += w4[u] * y[u][0];
-          o1 += w4[u] * y[u][1];
-        }
-      }
-    } else {
-      float M = kNegBig;
-      for (int c0 = 0; c0 < nc; c0 += kWave) {
-        if (c0 + lane < nc) M = fmaxf(M, a.ws_ml[(int64_t)merge_slot(a, glo, s0, glo + c0 + lane, kvh, h) * 2]);
-      }
-      M = wave_max(M);
-      for (int c0 = 0; c0 < nc; c0 += kWave) {
-        int my_slot = 0;
-        float wgt = 0.0f;
-        if (c0 + lane < nc) {
-          my_slot = merge_slot(a, glo, s0, glo + c0 + lane, kvh, h);
-          wgt = __builtin_amdgcn_exp2f(a.ws_ml[(int64_t)my_slot * 2] - M);
-          l += wgt * a.ws_ml[(int64_t)my_slot * 2 + 1];
-        }
-        const int cnt = nc - c0 < kWave ? nc - c0 : kWave;
-        int j = 0;
-        for (; j + 4 <= cnt; j += 4) {
-          f32x2 x[4];
-          float w4[4];
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            const int64_t sl = __builtin_amdgcn_readlane(my_slot, j + u);
-            w4[u] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wgt), j + u));
-            x[u] = *reinterpret_cast<const f32x2*>(a.ws_acc + sl * kHeadDim + 2 * lane);
-          }
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            o0 += w4[u] * x[u][0];
-            o1 += w4[u] * x[u][1];
-          }
-        }
-        for (; j < cnt; ++j) {
-          const int64_t sl = __builtin_amdgcn_readlane(my_slot, j);
-          const float w1 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wgt), j));
-          const f32x2 x = *reinterpret_cast<const f32x2*>(a.ws_acc + sl * kHeadDim + 2 * lane);
-          o0 += w1 * x[0];
-          o1 += w1 * x[1];
-        }
-      }
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) l += __shfl_xor(l, o);
+    merge_partials(a, 0, ghi - glo + 1, [&](int i) { return merge_slot(a, glo, s0, glo + i, kvh, h); }, o0, o1, l);
   }
   const float inv = l > 0.0f ? (kv_fp8 ? load_uniform_f32(a.v_scale) : 1.0f) / l : 0.0f;
   if (own) store_out2(a, off, o0 * inv, o1 * inv);
@@ -2357,21 +2657,20 @@ __global__ __launch_bounds__(kDecWaves* kWave) void paged_decode_stream_merge_ke
 // ---------------------------------------------------------------------------
 // fp32 KV kernel: v_mfma_f32_16x16x4_f32, 16-token tiles, same lane mapping.
 // ---------------------------------------------------------------------------
-template <bool PAIR>
-__global__ __launch_bounds__(kDecWaves* kWave) void paged_decode_mfma32_kernel(DecodeArgs a) {
+template <bool PAIR, bool SMALL>
+__global__ __launch_bounds__(kDecWaves* kWave) __attribute__((amdgpu_waves_per_eu(2))) void
+paged_decode_mfma32_kernel(DecodeArgs a) {
   WorkItem it;
   if (!decode_work_item(a, wave_work_index(), it)) return;
   float qf[32];
-  load_q_f32<PAIR>(a, it.b, it.kvh, qf);
-  const float score_mul = a.sm_scale * kLog2e;
-  f32x4 acc[8];
-#pragma unroll
-  for (int mm = 0; mm < 8; ++mm) acc[mm] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m_run = kNegBig, l_run = 0.0f;
-  f32_range(a, it, qf, score_mul, acc, m_run, l_run);
-  float l_col = l_run + __shfl_xor(l_run, 16);
-  l_col += __shfl_xor(l_col, 32);
-  finish_item<PAIR>(a, it, acc, m_run, l_col, 1.0f);
+  load_q_f32<PAIR, SMALL>(a, it.b, it.kvh, qf);
+  F32State<PAIR, SMALL> st;
+  f32_range<PAIR, SMALL>(a, it, qf, a.sm_scale * kLog2e, st);
+  f32_close<PAIR, SMALL>(st);
+  if constexpr (SMALL)
+    finish_item_f32_small<PAIR>(a, it, st);
+  else
+    finish_item<PAIR, true>(a, it, st.acc, st.m[0], st.l[0], 1.0f);
 }
 
 // ---------------------------------------------------------------------------
@@ -2389,17 +2688,8 @@ __global__ __launch_bounds__(kDecWaves* kWave) void paged_decode_merge_kernel(De
   L = L < 0 ? 0 : (L > cap ? cap : L);
   const int ns = L > 0 ? (int)((L + a.split_tokens - 1) / a.split_tokens) : 1;
   if (ns <= 1) return;
-  const int64_t slot0 = ((int64_t)b * a.num_heads + hq) * a.max_splits;
-  float M = kNegBig;
-  for (int s = 0; s < ns; ++s) M = fmaxf(M, a.ws_ml[(slot0 + s) * 2]);
-  float l = 0.0f, o0 = 0.0f, o1 = 0.0f;
-  for (int s = 0; s < ns; ++s) {
-    const float wgt = __builtin_amdgcn_exp2f(a.ws_ml[(slot0 + s) * 2] - M);
-    l += wgt * a.ws_ml[(slot0 + s) * 2 + 1];
-    const f32x2 x = *reinterpret_cast<const f32x2*>(a.ws_acc + (slot0 + s) * kHeadDim + 2 * lane);
-    o0 += wgt * x[0];
-    o1 += wgt * x[1];
-  }
+  float o0, o1, l;
+  merge_partials(a, ((int64_t)b * a.num_heads + hq) * a.max_splits, ns, [](int i) { return i; }, o0, o1, l);
   const float inv = l > 0.0f ? (kv_fp8 ? load_uniform_f32(a.v_scale) : 1.0f) / l : 0.0f;
   bool own;
   const int64_t off = (int64_t)b * a.out_stride + merge_out_offset(a, hq, hq % a.group, lane, own);
@@ -2414,15 +2704,24 @@ int ilog2_exact(int v) {
 }
 
 int default_split_tokens(int batch, int num_kv_heads, int max_blocks, int block_size) {
-  // Aim for >= ~4096 work items (256 CUs x 16 waves) so that the grid fills
-  // the chip even when the batch is small, but never split below 64 tokens.
+  // About 1024 work items (one wave per SIMD) from the longest context the
+  // table allows, in splits of 64 tokens or more: a wave's start-up and its
+  // partial cost as much as ~100 tokens.  At most 192 tokens, so that a batch
+  // of uneven lengths stays balanced, except where whole sequences already
+  // fill the chip (there 512, which bounds the workspace).  Measured on fp32
+  // caches, splits of 64 / 96 / 128 / 192 / 256 / 512 tokens: batch 1 of 700
+  // tokens 14.1 / 16.3 / 18.4 / 21.9 / 25.8 / 43.0 us; batch 8 of 1000-3000
+  // 38.2 / 34.5 / 39.2 / 29.9 / 31.7 / 47.7; batch 32 of 64-2048 48.8 / 46.1
+  // / 47.2 / 41.3 / 49.2 / 47.5; batch 200 of 20-2000 135 / 129 / 127 / 127 /
+  // 129 / 130.
   const int64_t items = (int64_t)batch * num_kv_heads;
   const int64_t max_len = (int64_t)max_blocks * block_size;
-  int64_t want_splits = (4096 + items - 1) / (items > 0 ? items : 1);
+  int64_t want_splits = (1024 + items - 1) / (items > 0 ? items : 1);
   int64_t st = (max_len + want_splits - 1) / (want_splits > 0 ? want_splits : 1);
   st = ((st + 31) / 32) * 32;
+  const int64_t most = items < 1024 ? 192 : 512;
   if (st < 64) st = 64;
-  if (st > 512) st = 512;
+  if (st > most) st = most;
   return (int)st;
 }
 
@@ -2488,6 +2787,9 @@ void launch_stream(DecodeArgs& a, int lds_bucket, size_t lds_bound, size_t lds, 
   hipLaunchKernelGGL(kernel, dim3(wgs), dim3(kDecWaves * kWave), lds, s, a);
 }
 
+// fp32 caches: the 4x4x1 MFMA form holds four query heads per cache head.
+bool f32_small_group(int group, bool pair) { return group <= (pair ? 8 : 4); }
+
 size_t split_ws_bytes(int batch, int num_heads, int max_blocks, int block_size, int st) {
   const int64_t max_splits = ((int64_t)max_blocks * block_size + st - 1) / st;
   if (max_splits <= 1) return 0;
@@ -2550,8 +2852,10 @@ int wg_waves(int batch, int kv_heads, int group, int max_blocks, int block_size,
 //     at most 128 tokens, whatever the batch; or at most 256 tokens when
 //     its waves also fill enough wave slots (items x waves >= 2 x CUs for
 //     per-tensor FP8, 6 x CUs for 16-bit caches, whose tiles are twice the
-//     bytes; per-token-head FP8 / INT8 never); fp32 caches: at most 512
-//     tokens with items x waves >= 2 x CUs.  Its time is set by the longest item's
+//     bytes; per-token-head FP8 / INT8 never); fp32 caches: items x
+//     waves >= 2 x CUs and at most 64 tokens a wave, or contexts of at most
+//     1024 tokens whose items give every CU one (at most 512 tokens a wave).
+//     Its time is set by the longest item's
 //     tile chain, so short contexts favour it and long ones do not.
 //     Measured (graph replays, 8 KV heads, FP8 / bf16 / FP8 per-token-head):
 //     batches 1 / 4 of 300-800 tokens in 4-block tables (128 tokens a wave)
@@ -2569,8 +2873,10 @@ int wg_waves(int batch, int kv_heads, int group, int max_blocks, int block_size,
 //     sizes for the larger of the two;
 //   * stream-K otherwise (16-bit / FP8 / INT8 caches): balanced over every
 //     wave whatever the lengths, at the cost of a merge launch;
-//   * split-K for fp32 caches otherwise (default split; the workgroup route
-//     took 37.0 us against 21.0 us for fp32 batch 4 of 207-798 tokens).
+//   * split-K for fp32 caches otherwise (default split).  Measured, fp32,
+//     workgroup against split-K: batch 1 of 200 tokens in a 512-token table
+//     12.9 against 13.9 us, of 700 in 768 19.7 against 14.1; batch 60 of 288-768 50.3 against 52.6; batch 32 of
+//     64-2048 46.5 against 41.3, batch 8 of 1000-3000 62.3 against 29.9.
 int choose_route(int split_tokens, int kv_dtype, int batch, const KernelShape& ks, int max_blocks,
                  int block_size, int cus, bool per_token = false) {
   if (split_tokens == MKV_DECODE_WORKGROUP) return kRouteWorkgroup;
@@ -2584,7 +2890,9 @@ int choose_route(int split_tokens, int kv_dtype, int batch, const KernelShape& k
   const int64_t fill = items * nw;
   bool wg;
   if (kv_dtype == MKV_DTYPE_F32)
-    wg = fill >= 2 * (int64_t)cus && wave_tokens <= 16 * kTileTok;
+    wg = fill >= 2 * (int64_t)cus && wave_tokens <= 16 * kTileTok &&
+         (wave_tokens <= 2 * kTileTok ||
+          (items >= cus && (int64_t)max_blocks * block_size <= 32 * kTileTok));
   else if (wave_tokens <= 4 * kTileTok)
     wg = true;
   else if (per_token || kv_dtype == MKV_DTYPE_I8)
@@ -2682,7 +2990,10 @@ int launch_route(DecodeArgs& a, int route, int fmt, int split_tokens, int max_bl
     }
     switch (fmt) {
       case MKV_DTYPE_F32:
-        hipLaunchKernelGGL(paged_decode_wg_f32_kernel<PAIR>, grid, block, lds, s, a);
+        if (f32_small_group(group, PAIR))
+          hipLaunchKernelGGL((paged_decode_wg_f32_kernel<PAIR, true>), grid, block, lds, s, a);
+        else
+          hipLaunchKernelGGL((paged_decode_wg_f32_kernel<PAIR, false>), grid, block, lds, s, a);
         break;
       case MKV_DTYPE_FP8E4M3:
         hipLaunchKernelGGL((paged_decode_wg_kernel<MKV_DTYPE_FP8E4M3, PAIR>), grid, block, lds, s, a);
@@ -2788,7 +3099,10 @@ int launch_route(DecodeArgs& a, int route, int fmt, int split_tokens, int max_bl
       hipLaunchKernelGGL((paged_decode_mfma16_kernel<MKV_DTYPE_F16, PAIR>), grid, block, 0, s, a);
       break;
     default:
-      hipLaunchKernelGGL(paged_decode_mfma32_kernel<PAIR>, grid, block, 0, s, a);
+      if (f32_small_group(group, PAIR))
+        hipLaunchKernelGGL((paged_decode_mfma32_kernel<PAIR, true>), grid, block, 0, s, a);
+      else
+        hipLaunchKernelGGL((paged_decode_mfma32_kernel<PAIR, false>), grid, block, 0, s, a);
       break;
   }
   if (a.max_splits > 1) {

@@ -367,3 +367,21 @@ def test_decode_default_route_block16_long_contexts(dev, dtype):
     for st in (0, WG):
         got = _run(dev, q, k, v, bt, ctx, 0.088, 16, 8, ks, vs, split_tokens=st)
         assert_close_out(got[idx], want, got.dtype, TOL[dtype])
+
+
+@pytest.mark.parametrize("route", [32, WG])
+@pytest.mark.parametrize("group", [1, 3, 4, 5])
+def test_decode_fp32_tiles_and_merge_edges(dev, group, route):
+    """fp32 caches on both matrix forms (at most four query heads per KV head,
+    and more), at lengths around the 16-token tile and around the split
+    merge's steps: 1, 4, 5, 12, 13, 64, 65 and 130 partials of 32 tokens.
+    Bound: a sum of n <= 4160 fp32 products of N(0, 1) values in any order
+    is within n ulps of its terms' sum; measured errors are 1e-6."""
+    announce(f"decode fp32 group {group}, tile and merge edges, route {route}")
+    parts = [1, 4, 5, 12, 13, 64, 65, 130]
+    ctx = torch.tensor([32 * n for n in parts] + [15, 16, 17, 32 * 64 + 1], dtype=torch.int64)
+    Hkv = 2
+    q, k, v, bt, ctx, ks, vs = _case(900 + group, len(ctx), Hkv * group, Hkv, 32, 440, 131, torch.float32, ctx=ctx)
+    got = _run(dev, q, k, v, bt, ctx, 1 / math.sqrt(128), Hkv * group, Hkv, split_tokens=route)
+    want = _oracle(q, k, v, bt, ctx, 1 / math.sqrt(128), Hkv * group, Hkv)
+    assert_close_out(got, want, got.dtype, 2e-5)

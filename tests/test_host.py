@@ -200,6 +200,26 @@ def test_decode_workspace_and_split_queries():
     assert lib.mkv_paged_decode_split_tokens(4, 8, 8, 256, 0) < st or st == 64
 
 
+def test_fp32_decode_route_and_split():
+    """fp32 caches: the workgroup route for short tables (64 tokens a wave,
+    two waves for every CU) and for contexts to 1024 tokens that give every CU an item; else split-K,
+    whose default split grows with the work until 192 tokens (512 where whole
+    sequences fill the chip)."""
+    lib = _lib.load()
+    SP, WG = _lib.ROUTE_SPLIT, _lib.ROUTE_WORKGROUP
+
+    def route(B, mb):
+        return lib.mkv_paged_decode_route(B, 16, 8, mb, 256, 128, _lib.DTYPE_F32, 0, 256)
+
+    assert route(7, 1) == SP and route(8, 1) == WG and route(8, 2) == WG and route(8, 3) == SP
+    assert route(31, 4) == SP and route(32, 4) == WG and route(32, 5) == SP and route(32, 8) == SP
+    assert lib.mkv_paged_decode_split_tokens(1, 8, 3, 256, 0) == 64
+    assert lib.mkv_paged_decode_split_tokens(8, 8, 12, 256, 0) == 192
+    assert lib.mkv_paged_decode_split_tokens(16, 8, 4, 256, 0) == 128
+    assert lib.mkv_paged_decode_split_tokens(32, 8, 16, 256, 0) == 192
+    assert lib.mkv_paged_decode_split_tokens(128, 8, 32, 256, 0) == 512
+
+
 def test_decode_route_choice():
     """The library's schedule for split_tokens 0 (mkv_paged_decode_route on
     a 256-CU device), for the decode workloads that are measured, and the
