@@ -410,7 +410,7 @@ struct WgWork {
 // tile list).  Returns false, uniformly over the workgroup, when it has no
 // tile.  Holds barriers: every thread of the workgroup must call it.
 template <bool PAGED>
-MKV_DEV bool wg_tile(const PrefillArgs& a, char* smem, WgWork& w) {
+MKV_DEV bool wg_tile(const PrefillArgs& a, char* list_lds, WgWork& w) {
   // XCD-aware order: with a multiple of 8 KV heads every XCD takes whole
   // heads (consecutive logical tiles share an XCD and its L2, and each XCD
   // sees the same longest-first mix); otherwise the tiles are dealt round
@@ -426,7 +426,7 @@ MKV_DEV bool wg_tile(const PrefillArgs& a, char* smem, WgWork& w) {
   int seq;
   int64_t q_seq0, q_seq1, tile, ctx;
   if (a.inline_list) {
-    TilePick& P = *reinterpret_cast<TilePick*>(smem + kTileListOffset);
+    TilePick& P = *reinterpret_cast<TilePick*>(list_lds);
     pick_tile_inline<PAGED>(a, P, tau, cap);
     if (P.seq < 0) return false;
     seq = P.seq;
@@ -478,11 +478,10 @@ MKV_DEV int row_vis_contiguous(const PrefillArgs& a, const WgWork& w, int row) {
   return (int)(v < w.ctx ? v : w.ctx);
 }
 
-// The number of keys each of the workgroup's kRowsPerWg rows sees, in
-// vis_lds[row] (0 for padding rows; paged), and their min / max over the real
-// rows.  Holds a barrier when paged: every thread of the workgroup must call
-// it.
-template <bool PAGED>
+// The number of keys each of the workgroup's ROWS rows sees, in vis_lds[row]
+// (0 for padding rows; paged), and their min / max over the real rows.  Holds
+// a barrier when paged: every thread of the workgroup must call it.
+template <bool PAGED, int ROWS>
 MKV_DEV void wg_rows(const PrefillArgs& a, int* vis_lds, int* red_lds, WgWork& w) {
   if constexpr (!PAGED) {
     // contiguous K/V: a row's visibility grows with its token, so the real
@@ -495,7 +494,8 @@ MKV_DEV void wg_rows(const PrefillArgs& a, int* vis_lds, int* red_lds, WgWork& w
   const int tid = threadIdx.x;
   const int64_t q0 = w.q0, q1 = w.q1, q_seq0 = w.q_seq0, ctx = w.ctx;
   const int G = a.group;
-  if (tid < kRowsPerWg) {
+  constexpr int kRowWaves = (ROWS + 63) / 64;
+  if (tid < 64 * kRowWaves) {
     const int64_t tok = q0 + tid / G;
     int vis = 0;
     if (tid < a.tok_per_wg * G && tok < q1) {
@@ -503,10 +503,10 @@ MKV_DEV void wg_rows(const PrefillArgs& a, int* vis_lds, int* red_lds, WgWork& w
       const int64_t v = pos + 1 < ctx ? pos + 1 : ctx;
       vis = v < 0 ? 0 : (int)v;
     }
-    vis_lds[tid] = vis;
-    // min / max over the real rows: the rows are waves 0 and 1; each reduces
-    // its 64 with lane shuffles and writes one pair (LDS atomics from every
-    // row to one address serialise: ~7 us per workgroup)
+    if (ROWS % 64 == 0 || tid < ROWS) vis_lds[tid] = vis;
+    // min / max over the real rows: the rows are the first kRowWaves waves;
+    // each reduces its 64 with lane shuffles and writes one pair (LDS atomics
+    // from every row to one address serialise: ~7 us per workgroup)
     const bool real = tid < a.tok_per_wg * G && tok < q1;
     int mn = real ? vis : 0x7fffffff, mx = real ? vis : 0;
 #pragma unroll
@@ -520,8 +520,13 @@ MKV_DEV void wg_rows(const PrefillArgs& a, int* vis_lds, int* red_lds, WgWork& w
     }
   }
   __syncthreads();
-  w.min_vis = min(red_lds[0], red_lds[2]);
-  w.max_vis = max(red_lds[1], red_lds[3]);
+  static_assert(kRowWaves <= 2, "red_lds holds two pairs");
+  w.min_vis = red_lds[0];
+  w.max_vis = red_lds[1];
+  if constexpr (kRowWaves == 2) {
+    w.min_vis = min(w.min_vis, red_lds[2]);
+    w.max_vis = max(w.max_vis, red_lds[3]);
+  }
 }
 
 // LDS geometry of one K or V tile: kBN key rows of 256 bytes (128 16-bit
@@ -601,7 +606,7 @@ MKV_DEV void prefill_mfma_body(const PrefillArgs& a) {
   // workgroup on the CU (raised to 1 below) do not hold them back.
   __builtin_amdgcn_s_setprio(3);
   WgWork wk;
-  if (!wg_tile<PAGED>(a, smem, wk)) return;
+  if (!wg_tile<PAGED>(a, smem + kTileListOffset, wk)) return;
   const int kvh = wk.kvh, seq = wk.seq;
   // (uniform: in scalar registers, not held in vector registers across the
   // key loop for the epilogue)
@@ -665,7 +670,7 @@ MKV_DEV void prefill_mfma_body(const PrefillArgs& a) {
   // head pairing: this lane's row belongs to the pair's second KV head
   const bool row_hi = PAIR && (kRowTiles * wave * 16 + c) % G >= (G >> 1);
   if constexpr (QSPLIT) convert_q();
-  wg_rows<PAGED>(a, vis_lds, red_lds, wk);
+  wg_rows<PAGED, kRowsPerWg>(a, vis_lds, red_lds, wk);
   const int min_vis = wk.min_vis, max_vis = wk.max_vis;
   int vis_c[kRowTiles];
 #pragma unroll
@@ -1368,20 +1373,35 @@ constexpr bool kPrefill2w = kPerTokenScale<KV_DT> && (QSPLIT || PAIR);
 // ---------------------------------------------------------------------------
 // fp32 caches (the reference engine's default precision, model_runner.py:87,
 // :249; flash_attention_prefill / paged_attention_prefill_triton take fp32,
-// attention.py:446-514, :852-891).  The same work decomposition as
-// prefill_mfma_kernel (128 rows of one sequence and KV head per workgroup,
-// the same tile list), on the fp32 MFMA (v_mfma_f32_16x16x4_f32: products
+// attention.py:446-514, :852-891).  The same tile list as
+// prefill_mfma_kernel, on the fp32 MFMA (v_mfma_f32_16x16x4_f32: products
 // and sums in fp32, no rounding of K, V, q or P below fp32).
 //
+// Bound by that MFMA (154 TFLOP/s in a large matrix product here): a wave's
+// 16 rows and 16 keys are 64 MFMAs of 32 cycles, against ~100 VALU and 16 LDS
+// instructions.  With 128 rows a workgroup a step of six ragged chunks behind
+// 0-2048 cached tokens (16 q / 8 kv heads) was 232 workgroups whose longest
+// kept two waves a SIMD busy for 80 tiles: 311 us, a quarter of the MFMA
+// rate.  A workgroup is now four waves, one a SIMD, in one of two forms:
+//   RT = 2: 32 rows; the two waves of a row tile take one 16-key sub-tile
+//     each of every 32-key tile and join their sums at the end.  A quarter of
+//     the rows and half the keys in a chain: 311 -> 145 us on that step.
+//   RT = 4: 64 rows, both sub-tiles by every wave, half the workgroups and no
+//     join: for launches with workgroups to spare (36 prompts of 46-478
+//     tokens, 32 / 8 heads: 177 us with 128 rows, 187 with RT 2, 168).
+//
 // Tiles of kBN32 = 32 keys x 512 bytes go from HBM straight into LDS by DMA
-// (buffer_load ... lds), double-buffered.  Wave w loads 8 consecutive keys
-// of one 16-key sub-tile: K (w < 4) or V, sub-tile (w % 4) / 2, keys
-// 8 (w % 2) .. +7, two key rows per instruction.  K rows are stored with
-// 16-byte chunk p holding logical chunk p ^ (key & 15) (the swizzle moves to
-// the global side of the DMA), so that the 16 lanes of a QK operand read
-// (16 keys, one logical chunk) hit 16 distinct chunk positions mod 16; V rows
-// are stored as they are (the 16 lanes of a PV operand read take one key's
-// chunks c and 16 + c).
+// (buffer_load ... lds), into a ring of three 16 KB slots: K of tile i + 1 is
+// requested at the start of tile i into the slot of V i - 1, V i + 1 after
+// QK i into the slot of K i, so each load has a whole tile's time and three
+// workgroups fit a CU (two K and two V buffers: two; 2 prompts of 215-774
+// tokens 61 -> 53 us, a 5-prompt prefill of 7 GFLOP 178 -> 162).  Every wave
+// loads 8 consecutive keys of a tile, two key rows per instruction.  K rows
+// are stored with 16-byte chunk p holding logical chunk p ^ (key & 15) (the
+// swizzle moves to the global side of the DMA), so that the 16 lanes of a QK
+// operand read (16 keys, one logical chunk) hit 16 distinct chunk positions
+// mod 16; V rows are stored as they are (the 16 lanes of a PV operand read
+// take one key's chunks c and 16 + c).
 //
 // Per wave (16 rows), per 16-key sub-tile kt:
 //   S^T = K Q^T: 32 MFMAs; lane (c, kg) supplies K[key c][32 kg + st] and
@@ -1392,30 +1412,61 @@ constexpr bool kPrefill2w = kPerTokenScale<KV_DT> && (QSPLIT || PAIR);
 //     lane column c hold dim 4c + mm (mm < 4) or 64 + 4c + mm - 4.
 // ---------------------------------------------------------------------------
 constexpr int kBN32 = 32;
+constexpr int kPfWaves32 = 4;
+constexpr int kPfThreads32 = kPfWaves32 * kWave;
+static_assert(kPfThreads32 >= kInlineSeqs, "pick_tile_inline takes a thread per sequence");
+
+// Workgroup barrier that leaves the LDS DMA in flight alone (__syncthreads
+// waits for all of it): this wave's LDS reads are done, its DMA is waited for
+// by count.
+MKV_DEV void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// s_waitcnt vmcnt(N) alone (the other counters at their maxima)
+template <int N>
+MKV_DEV void vm_wait() {
+  static_assert(N < 16, "the low field of vmcnt");
+  __builtin_amdgcn_s_waitcnt(0x0f70 | N);
+}
 constexpr int kRowBytes32 = kHeadDim * 4;          // 512
 constexpr int kTileBytes32 = kBN32 * kRowBytes32;  // 16 KB per K or V tile
+// dynamic LDS: row visibility [16 RT] + 4 ints, then the inline tile list
+template <int RT>
+constexpr int kTileListOffset32 = (16 * RT + 4) * 4;
+static_assert(kTileListOffset32<4> % 8 == 0, "TilePick holds 64-bit fields");
+// three workgroups a CU (160 KB of LDS, handed out in 1280-byte units)
+static_assert(3 * ((3 * kTileBytes32 + kTileListOffset32<4> + (int)sizeof(TilePick) + 1279) / 1280) <= 128,
+              "three workgroups a CU");
 
-template <bool PAGED, bool PAIR>
-__global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(4))) void prefill_f32_kernel(PrefillArgs a) {
+template <bool PAGED, bool PAIR, int RT>
+__global__ __launch_bounds__(kPfThreads32) __attribute__((amdgpu_waves_per_eu(3))) void prefill_f32_kernel(PrefillArgs a) {
+  constexpr int kRows = 16 * RT;
+  constexpr int kKeyHalves = kPfWaves32 / RT;  // waves of a row tile
+  constexpr int kSubs = 2 / kKeyHalves;        // 16-key sub-tiles of a wave, per tile
   extern __shared__ __align__(16) char smem[];
-  __shared__ __align__(16) char lds_k0[kTileBytes32], lds_v0[kTileBytes32], lds_k1[kTileBytes32],
-      lds_v1[kTileBytes32];
+  __shared__ __align__(16) char lds_0[kTileBytes32], lds_1[kTileBytes32], lds_2[kTileBytes32];
   int* vis_lds = reinterpret_cast<int*>(smem);
-  int* red_lds = vis_lds + kRowsPerWg;
+  int* red_lds = vis_lds + kRows;
 
   const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, kg = lane >> 4;
+  const int rt = wave % RT;  // row tile
+  const int kt = wave / RT;  // its sub-tile of every tile (kKeyHalves 2; else both)
 
   WgWork wk;
-  if (!wg_tile<PAGED>(a, smem, wk)) return;
+  if (!wg_tile<PAGED>(a, smem + kTileListOffset32<RT>, wk)) return;
   const int kvh = wk.kvh, seq = wk.seq;
-  const int64_t q0 = wk.q0, q1 = wk.q1;
+  // (uniform: in scalar registers)
+  const int64_t q_seq0 = uniform_i64(wk.q_seq0), q0 = uniform_i64(wk.q0), q1 = uniform_i64(wk.q1);
   const int G = a.group;
 
   // q of row c (dims 32 kg .. 32 kg + 31), fp32, loaded before the rows'
   // visibility is worked out
-  const int my_row = 16 * wave + c;
+  const int my_row = 16 * rt + c;
   float qf[32];
   {
     const int64_t tok = q0 + my_row / G;
@@ -1431,8 +1482,9 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(4)))
       for (int i = 0; i < 32; ++i) qf[i] = 0.0f;
     }
   }
-  wg_rows<PAGED>(a, vis_lds, red_lds, wk);
-  const int min_vis = wk.min_vis, max_vis = wk.max_vis;
+  wg_rows<PAGED, kRows>(a, vis_lds, red_lds, wk);
+  const int min_vis = __builtin_amdgcn_readfirstlane(wk.min_vis);
+  const int max_vis = __builtin_amdgcn_readfirstlane(wk.max_vis);
   const int vis_row = PAGED ? vis_lds[my_row] : row_vis_contiguous(a, wk, my_row);
   // The loop keeps raw scores and needs score_mul > 0 (as prefill_mfma_kernel).
   float score_mul = a.sm_scale * kLog2e;
@@ -1448,104 +1500,131 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(4)))
   for (int mm = 0; mm < 8; ++mm) acc[mm] = f32x4{0.f, 0.f, 0.f, 0.f};
   float m_run = kNegBig, l_run = 0.0f;
 
-  // DMA geometry of this wave: tensor (K for waves 0-3), sub-tile j, first
-  // key kw of its 8; lane l fills key kw + 2u + l / 32 at chunk position
-  // l % 32 in instruction u.
+  // DMA geometry: each wave loads 32 / 4 consecutive keys of a K or V tile,
+  // two rows an instruction; lane l fills key 2u + l / 32 of them at chunk
+  // position l % 32 in instruction u.
+  constexpr int kDmaKeys = kBN32 / kPfWaves32, kDmas = kDmaKeys / 2;
   const int64_t row_stride = (int64_t)a.num_kv_heads * kRowBytes32;
   const int64_t head_bytes = (int64_t)kvh * kRowBytes32;
-  const bool w_is_v = wave >= 4;
-  const int w_sub = (wave & 3) >> 1;
-  const int w_key = 8 * (wave & 1);
-  uint32_t dma_off[4];
+  const int w_key = wave * kDmaKeys;  // within the tile
+  uint32_t dma_off_k[kDmas], dma_off_v[kDmas];
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int key = w_key + 2 * u + (lane >> 5);  // within the sub-tile (== key & 15)
+  for (int u = 0; u < kDmas; ++u) {
+    const int key = (w_key + 2 * u + (lane >> 5)) & 15;  // within the sub-tile
     const int p = lane & 31;
-    const int gch = w_is_v ? p : (p ^ key);
-    dma_off[u] = (uint32_t)(key * row_stride + 16 * gch);
+    dma_off_k[u] = (uint32_t)(key * row_stride + 16 * (p ^ key));
+    dma_off_v[u] = (uint32_t)(key * row_stride + 16 * p);
   }
-  auto dma_tile = [&](int kb, char* kbuf, char* vbuf) {
-    const int64_t t0 = kb + 16 * w_sub;
-    const char* base = w_is_v ? a.v : a.k;
-    const char* ptr = base;
-    int num = 0;
+  // Block-table entries of a tile, read a tile ahead of its DMA (lane l: the
+  // entry of sub-tile l / 32, -1 when absent): a lookup at its use would wait
+  // for the tile's DMA too, since both count in vmcnt.
+  auto entry_load = [&](int kb) -> int {
     if constexpr (PAGED) {
-      const int64_t phys = a.idx.physical_block(seq, t0 >> a.idx.bs_log2);
-      if (phys >= 0) {
+      const int blk = (kb + 16 * (lane >> 5)) >> a.idx.bs_log2;
+      return a.idx.block_tables[(int64_t)seq * a.idx.bt_stride + (blk < a.idx.max_blocks ? blk : 0)];
+    } else {
+      return 0;
+    }
+  };
+  const uint32_t num_blocks32 = PAGED ? (uint32_t)min(a.idx.num_blocks, (int64_t)0x7fffffff) : 1u;
+  auto dma_tile = [&](int kb, int ent, const char* base, const uint32_t* dma_off, char* buf) {
+    const int t0 = kb + (w_key & 16);
+    const char* ptr = base;
+    int num = (int)(15 * row_stride + kRowBytes32);
+    if constexpr (PAGED) {
+      const int phys = __builtin_amdgcn_readlane(ent, 2 * (w_key & 16));
+      if ((uint32_t)phys < num_blocks32) {
         const int64_t bmask = ((int64_t)1 << a.idx.bs_log2) - 1;
-        ptr = base + ((phys << a.idx.bs_log2) + (t0 & bmask)) * row_stride + head_bytes;
-        num = (int)(15 * row_stride + kRowBytes32);
+        ptr += (((int64_t)phys << a.idx.bs_log2) + (t0 & bmask)) * row_stride + head_bytes;
+      } else {
+        num = 0;
       }
     } else {
-      ptr = base + (wk.q_seq0 + t0) * row_stride + head_bytes;
-      num = (int)(15 * row_stride + kRowBytes32);
+      ptr += (q_seq0 + t0) * row_stride + head_bytes;
     }
     const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)ptr, (short)0, num, 0x00020000);
-    char* dst0 = (w_is_v ? vbuf : kbuf) + (16 * w_sub + w_key) * kRowBytes32;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int64_t key = t0 + w_key + 2 * u + (lane >> 5);
+    for (int u = 0; u < kDmas; ++u) {
+      const int key = kb + w_key + 2 * u + (lane >> 5);
       const uint32_t off = key < max_vis ? dma_off[u] : 0x80000000u;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          r, (__attribute__((address_space(3))) void*)(dst0 + 2 * u * kRowBytes32), 16, off, 0, 0, 0);
+          r, (__attribute__((address_space(3))) void*)(buf + (w_key + 2 * u) * kRowBytes32), 16, off, 0, 0, 0);
     }
   };
-  // validity of the two 16-key sub-tiles of the tile at kb (absent blocks)
-  auto sub_valid = [&](int kb, int kt) -> bool {
-    if constexpr (PAGED) return a.idx.physical_block(seq, (int64_t)(kb + 16 * kt) >> a.idx.bs_log2) >= 0;
-    return true;
-  };
-
   const int n_tiles = (max_vis + kBN32 - 1) / kBN32;
   const bool wave_active = __builtin_amdgcn_ballot_w64(vis_row > 0) != 0;
-  if (n_tiles > 0) {
-    dma_tile(0, lds_k0, lds_v0);
-    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
-  }
-  __syncthreads();
-  for (int it0 = 0; it0 < n_tiles; it0 += 2) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int it = it0 + h;
-      if (it >= n_tiles) break;
-      char* kbuf = h ? lds_k1 : lds_k0;
-      char* vbuf = h ? lds_v1 : lds_v0;
+  // Tile `it` in ring slots kbuf, vbuf; K of the next tile goes to the slot
+  // vfree of the V tile before, V of the next to kbuf once every wave is done
+  // with it.  The loads past the last tile read no memory (every key is past
+  // max_vis) and are issued all the same: the waits count loads, and the
+  // compiler's own count (for the entries and the LDS reads) has to see the
+  // same loads on every path.
+  auto tile_step = [&](int it, char* kbuf, char* vbuf, char* vfree, int e_cur, int e_next, int& e_ahead) {
       const int kb = it * kBN32;
-      if (it + 1 < n_tiles) dma_tile(kb + kBN32, h ? lds_k0 : lds_k1, h ? lds_v0 : lds_v1);
-      if (wave_active) {
-        bool kvalid[2];
+      // K of this tile has landed (V's loads are the only later ones)
+      vm_wait<kDmas>();
+      lds_barrier();
+      dma_tile(kb + kBN32, e_next, a.k, dma_off_k, vfree);
+      e_ahead = entry_load(kb + 2 * kBN32);
+      const int k0 = kb + 16 * kt;  // this wave's first key
+      const bool active = wave_active && k0 < max_vis;
+      f32x4 s[kSubs];
+      if (active) {
+        // ---- S^T = K Q^T, in two accumulators (half the dependent chain) ----
 #pragma unroll
-        for (int kt = 0; kt < 2; ++kt) kvalid[kt] = sub_valid(kb, kt);
-        const bool full = kb + kBN32 <= min_vis && kvalid[0] && kvalid[1];
-        // ---- S^T = K Q^T ----
-        f32x4 s[2];
+        for (int j = 0; j < kSubs; ++j) {
+          const char* krow = kbuf + (16 * (kt + j) + c) * kRowBytes32;
+          f32x4 kf[8];
 #pragma unroll
-        for (int kt = 0; kt < 2; ++kt) {
-          s[kt] = f32x4{0.f, 0.f, 0.f, 0.f};
-          const char* krow = kbuf + (16 * kt + c) * kRowBytes32;
+          for (int qd = 0; qd < 8; ++qd) kf[qd] = *reinterpret_cast<const f32x4*>(krow + 16 * ((8 * kg + qd) ^ c));
+          __builtin_amdgcn_sched_barrier(0);
+          f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int qd = 0; qd < 8; ++qd) {
-            const f32x4 kv4 = *reinterpret_cast<const f32x4*>(krow + 16 * ((8 * kg + qd) ^ c));
+          for (int qd = 0; qd < 8; ++qd)
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-              s[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv4[e], qf[4 * qd + e], s[kt], 0, 0, 0);
-          }
+            for (int e = 0; e < 4; e += 2) {
+              s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[qd][e], qf[4 * qd + e], s0, 0, 0, 0);
+              s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[qd][e + 1], qf[4 * qd + e + 1], s1, 0, 0, 0);
+            }
+#pragma unroll
+          for (int r = 0; r < 4; ++r) s[j][r] = s0[r] + s1[r];
         }
+      }
+      // V of this tile has landed, and every wave is done with K
+      vm_wait<kDmas + (PAGED ? 1 : 0)>();
+      lds_barrier();
+      dma_tile(kb + kBN32, e_next, a.v, dma_off_v, kbuf);
+      if (active) {
+        bool valid[kSubs];  // sub-tiles in a present block
+        bool full = k0 + 16 * kSubs <= min_vis;
+#pragma unroll
+        for (int j = 0; j < kSubs; ++j) {
+          valid[j] = !PAGED || (uint32_t)__builtin_amdgcn_readlane(e_cur, 32 * (kt + j)) < num_blocks32;
+          full = full && valid[j];
+        }
+        // V of keys 4 kg + r of a sub-tile, the first two ahead of the softmax
+        const char* vrow = vbuf + (16 * kt + 4 * kg) * kRowBytes32 + 16 * c;
+        f32x4 v_lo[4], v_hi[4];
+        auto v_load = [&](int j, int r) {
+          v_lo[r] = *reinterpret_cast<const f32x4*>(vrow + (16 * j + r) * kRowBytes32);
+          v_hi[r] = *reinterpret_cast<const f32x4*>(vrow + (16 * j + r) * kRowBytes32 + 256);
+        };
+        v_load(0, 0);
+        v_load(0, 1);
+        __builtin_amdgcn_sched_barrier(0);
         // ---- online softmax (log2 domain) for row c ----
         if (!full) {
 #pragma unroll
-          for (int kt = 0; kt < 2; ++kt)
+          for (int j = 0; j < kSubs; ++j)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const int t = kb + 16 * kt + 4 * kg + r;
-              if (!(t < vis_row && kvalid[kt])) s[kt][r] = -__builtin_huge_valf();
-            }
+            for (int r = 0; r < 4; ++r)
+              if (!(k0 + 16 * j + 4 * kg + r < vis_row && valid[j])) s[j][r] = -__builtin_huge_valf();
         }
         float mx = -__builtin_huge_valf();
 #pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
+        for (int j = 0; j < kSubs; ++j)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[kt][r]);
+          for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[j][r]);
         mx = max_xor32(max_xor16(mx));
         mx = fmaxf(mx * score_mul, kNegBig);
         const float m_new = mx > m_run + kRescaleSlack ? mx : m_run;
@@ -1553,11 +1632,11 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(4)))
         m_run = m_new;
         float psum = 0.0f;
 #pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
+        for (int j = 0; j < kSubs; ++j)
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            s[kt][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kt][r], score_mul, -m_new));
-            psum += s[kt][r];
+            s[j][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[j][r], score_mul, -m_new));
+            psum += s[j][r];
           }
         l_run = l_run * alpha + psum;
         if (__builtin_amdgcn_ballot_w64(alpha != 1.0f)) {
@@ -1570,21 +1649,65 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(4)))
         }
         // ---- O += P V ----
 #pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
+        for (int j = 0; j < kSubs; ++j) {
+          if (j) {
+            v_load(j, 0);
+            v_load(j, 1);
+          }
+          v_load(j, 2);
+          v_load(j, 3);
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const char* vrow = vbuf + (16 * kt + 4 * kg + r) * kRowBytes32;
-            const f32x4 v_lo = *reinterpret_cast<const f32x4*>(vrow + 16 * c);
-            const f32x4 v_hi = *reinterpret_cast<const f32x4*>(vrow + 256 + 16 * c);
+          for (int r = 0; r < 4; ++r)
 #pragma unroll
             for (int mm = 0; mm < 4; ++mm) {
-              acc[mm] = __builtin_amdgcn_mfma_f32_16x16x4f32(s[kt][r], v_lo[mm], acc[mm], 0, 0, 0);
-              acc[4 + mm] = __builtin_amdgcn_mfma_f32_16x16x4f32(s[kt][r], v_hi[mm], acc[4 + mm], 0, 0, 0);
+              acc[mm] = __builtin_amdgcn_mfma_f32_16x16x4f32(s[j][r], v_lo[r][mm], acc[mm], 0, 0, 0);
+              acc[4 + mm] = __builtin_amdgcn_mfma_f32_16x16x4f32(s[j][r], v_hi[r][mm], acc[4 + mm], 0, 0, 0);
             }
-          }
-      }  // wave_active
-      __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's DMA has landed
-      __syncthreads();
+        }
+      }
+  };
+  int e0 = 0, e1 = 0, e2 = 0;  // entries of tiles 0, 1, 2 mod 3
+  if (n_tiles > 0) {
+    e0 = entry_load(0);
+    e1 = entry_load(kBN32);
+    dma_tile(0, e0, a.k, dma_off_k, lds_0);
+    dma_tile(0, e0, a.v, dma_off_v, lds_1);
+  }
+  for (int it = 0; it < n_tiles; it += 3) {
+    tile_step(it, lds_0, lds_1, lds_2, e0, e1, e2);
+    if (it + 1 < n_tiles) tile_step(it + 1, lds_2, lds_0, lds_1, e1, e2, e0);
+    if (it + 2 < n_tiles) tile_step(it + 2, lds_1, lds_2, lds_0, e2, e0, e1);
+  }
+  vm_wait<0>();
+  __syncthreads();
+
+  // ---- the two key halves of a row tile, joined through LDS ----
+  if constexpr (kKeyHalves == 2) {
+    constexpr int kXs = 64 * RT;
+    static_assert(32 * kXs * 4 <= kTileBytes32, "the row tiles' accumulators fit one slot");
+    float* x_acc = reinterpret_cast<float*>(lds_0) + 64 * rt + lane;  // [32][row tile][lane]
+    float* x_ml = reinterpret_cast<float*>(lds_1) + 64 * rt + lane;   // [2][row tile][lane]
+    if (kt == 1) {
+#pragma unroll
+      for (int mm = 0; mm < 8; ++mm)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x_acc[(4 * mm + r) * kXs] = acc[mm][r];
+      x_ml[0] = m_run;
+      x_ml[kXs] = l_run;
+    }
+    __syncthreads();
+    if (kt == 1) return;
+    {
+      const float m1 = x_ml[0];
+      const float m = fmaxf(m_run, m1);
+      const float f0 = __builtin_amdgcn_exp2f(m_run - m), f1 = __builtin_amdgcn_exp2f(m1 - m);
+      l_run = l_run * f0 + x_ml[kXs] * f1;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float g0 = __shfl(f0, 4 * kg + r), g1 = __shfl(f1, 4 * kg + r);
+#pragma unroll
+        for (int mm = 0; mm < 8; ++mm) acc[mm][r] = acc[mm][r] * g0 + x_acc[(4 * mm + r) * kXs] * g1;
+      }
     }
   }
 
@@ -1599,7 +1722,7 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(4)))
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const float lh = __shfl(l_col, 4 * kge + r);
-    const int row = 16 * wave + 4 * kge + r;
+    const int row = 16 * rt + 4 * kge + r;
     const int rq = (int)(((uint32_t)row * gm) >> 16), rm = row - rq * G;
     const int64_t tok = q0 + rq;
     if (row >= a.tok_per_wg * G || tok >= q1) continue;
@@ -1644,11 +1767,8 @@ int ilog2_exact(int v) {
   return l;
 }
 
-int tok_per_wg_for(int group) { return kRowsPerWg / group; }
-
-int64_t tiles_upper_bound(int num_seqs, int64_t total_q, int group) {
-  const int tpw = tok_per_wg_for(group);
-  return (total_q + tpw - 1) / tpw + num_seqs;
+int64_t tiles_upper_bound(int num_seqs, int64_t total_q, int tok_per_wg) {
+  return (total_q + tok_per_wg - 1) / tok_per_wg + num_seqs;
 }
 
 template <int KV_DT, bool PAGED, bool QSPLIT>
@@ -1674,15 +1794,37 @@ int launch_prefill(const PrefillArgs& a, hipStream_t s) {
   return (int)hipGetLastError();
 }
 
-template <bool PAGED>
+// fp32 launches, by the number of 32-row workgroups they make:
+//  * 4096 or more (five rounds of three a CU): 64 rows a workgroup.  5750
+//    (25 prompts of 55-596 tokens): 180 -> 162 us; 3000 (5 prompts of
+//    106-1489): 162 / 161; 2100 (6 of 25-1330): 106 -> 124, a longer last
+//    round.
+//  * under three a CU: two workgroups a CU, by LDS they do not use.  All of
+//    them start at once, and a CU dealt three long ones ends last (435 of
+//    four chunks behind 1175-3816 tokens: 239 us at two a CU, 274 at three;
+//    513 of two chunks: 142 / 157); from 768 on the third hides more than
+//    that costs (810: 236 / 208).
+constexpr int64_t kF32Wide = 4096, kF32Dense = 768;
+constexpr size_t kF32SparseLds = 8192;
+static_assert(2 * (3 * kTileBytes32 + 8192 + 4096) <= 160 * 1024 && 3 * (3 * kTileBytes32 + 8192) > 160 * 1024,
+              "two workgroups a CU");
+
+int64_t f32_small_wgs(const PrefillArgs& a) {
+  const int tpw = 32 / a.group;
+  return (a.total_q + tpw - 1) / tpw * a.num_kv_heads;
+}
+
+template <bool PAGED, int RT>
 int launch_prefill_f32(const PrefillArgs& a, hipStream_t s) {
-  const size_t lds = kTileListOffset + (a.inline_list ? sizeof(TilePick) : 0);
+  const size_t lds = kTileListOffset32<RT> + (a.inline_list ? sizeof(TilePick) : 0) +
+                     (f32_small_wgs(a) < kF32Dense ? kF32SparseLds : 0);
   int64_t nwg = a.tiles_ub * a.num_kv_heads;
   nwg = ((nwg + kXcds - 1) / kXcds) * kXcds;
+  const dim3 grid((unsigned)nwg), block(kPfThreads32);
   if (a.pair)
-    hipLaunchKernelGGL((prefill_f32_kernel<PAGED, true>), dim3((unsigned)nwg), dim3(kPfThreads), lds, s, a);
+    hipLaunchKernelGGL((prefill_f32_kernel<PAGED, true, RT>), grid, block, lds, s, a);
   else
-    hipLaunchKernelGGL((prefill_f32_kernel<PAGED, false>), dim3((unsigned)nwg), dim3(kPfThreads), lds, s, a);
+    hipLaunchKernelGGL((prefill_f32_kernel<PAGED, false, RT>), grid, block, lds, s, a);
   return (int)hipGetLastError();
 }
 
@@ -1739,8 +1881,10 @@ int dispatch_prefill(PrefillArgs& a, int kv_dtype, void* workspace, size_t works
   a.tile_start = reinterpret_cast<int32_t*>(workspace);
   int32_t* order = a.tile_start + a.num_seqs + 1;
   a.order = order;
-  a.tok_per_wg = tok_per_wg_for(a.group);
-  a.tiles_ub = tiles_upper_bound(a.num_seqs, a.total_q, a.group);
+  const bool f32 = kv_dtype == MKV_DTYPE_F32;
+  const int f32_rt = f32 && f32_small_wgs(a) >= kF32Wide ? 4 : 2;
+  a.tok_per_wg = (f32 ? 16 * f32_rt : kRowsPerWg) / a.group;
+  a.tiles_ub = tiles_upper_bound(a.num_seqs, a.total_q, a.tok_per_wg);
   a.inline_list = a.num_seqs <= kInlineSeqs;
   if (!a.inline_list) {
     const int64_t ctx_cap = PAGED ? ((int64_t)a.idx.max_blocks << a.idx.bs_log2) : 0;
@@ -1752,7 +1896,8 @@ int dispatch_prefill(PrefillArgs& a, int kv_dtype, void* workspace, size_t works
   // fp16 after its power-of-two normalisation, an fp32 q takes two terms
   const bool q16 = a.q_dtype != MKV_DTYPE_F32;
   switch (kv_dtype) {
-    case MKV_DTYPE_F32: return launch_prefill_f32<PAGED>(a, s);
+    case MKV_DTYPE_F32:
+      return f32_rt == 4 ? launch_prefill_f32<PAGED, 4>(a, s) : launch_prefill_f32<PAGED, 2>(a, s);
     case MKV_DTYPE_FP8E4M3: return launch_prefill<MKV_DTYPE_FP8E4M3, PAGED, false>(a, s);
     case kKvFp8PerToken:
       if constexpr (PAGED)

@@ -533,3 +533,35 @@ def test_attention_layer_fp32_auto_full_then_chunked_then_decode(dev):
     step([20, 1, 64], full=False)
     step([1, 1, 1], full=False)
     step([1, 0, 1], full=False)
+
+
+@pytest.mark.parametrize("paged", [True, False])
+@pytest.mark.parametrize("Hkv,group,copies", [(2, 1, 1), (2, 3, 2), (4, 4, 16), (8, 4, 12), (8, 16, 16)])
+def test_prefill_fp32_workgroup_forms(dev, paged, Hkv, group, copies):
+    """fp32 caches in every launch form (few 32-row workgroups, three a CU,
+    64 rows each), with lengths around the 16- and 32-key tiles, the ring of
+    three and the rows of a workgroup, and an absent block.  Bound: a sum of
+    n <= 260 fp32 products of N(0, 1) values in any order is within n ulps
+    of its terms' sum; measured errors are 1e-6."""
+    announce(f"prefill fp32 forms paged {paged} {Hkv} x {group} x {copies}")
+    qlen = [1, 2, 15, 16, 17, 31, 33, 64, 65, 97, 130]
+    prior = [0, 31, 1, 16, 15, 0, 95, 0, 31, 0, 130] if paged else [0] * len(qlen)
+    holes = [(10, 5)] if paged else []
+    q, k, v, bt, ctx, cu, pos, _, _ = _make(77, prior, qlen, Hkv * group, Hkv, 16, torch.float32, holes=holes)
+    sc = 1 / math.sqrt(128)
+    n, T = len(qlen), q.shape[0]
+    if paged:
+        want = R.paged_prefill_ref(q.double(), k, v, bt, ctx, cu, pos, sc, Hkv * group, Hkv, None, None)
+    else:
+        k, v = k.flatten(0, 1)[:T], v.flatten(0, 1)[:T]
+        want = R.flash_prefill_ref(q.double(), k.double(), v.double(), cu, sc, Hkv * group, Hkv)
+    # the batch repeated `copies` times over one pool
+    off = torch.arange(copies, dtype=torch.int32).repeat_interleave(n) * T
+    cu = torch.cat([cu[:-1].repeat(copies) + off, torch.tensor([copies * T], dtype=torch.int32)])
+    if paged:
+        got = _gpu(dev, q.repeat(copies, 1, 1), k, v, bt.repeat(copies, 1), ctx.repeat(copies), cu,
+                   pos.repeat(copies), sc, Hkv * group, Hkv, None, None)
+    else:
+        got = A.flash_attention_prefill(q.repeat(copies, 1, 1).to(dev), k.repeat(copies, 1, 1).to(dev),
+                                        v.repeat(copies, 1, 1).to(dev), cu.to(dev), sc, Hkv * group, Hkv, 128).cpu()
+    assert_close_out(got, want.repeat(copies, 1, 1), got.dtype, 2e-5)
