@@ -526,6 +526,20 @@ int mkv_rmsnorm(void* out, void* residual, const void* x, const void* weight,
 int mkv_silu_mul(void* out, const void* x, int64_t x_row_stride, int64_t rows,
                  int inter, int dtype, void* stream);
 
+/* out = x w^T for at most 64 rows of x: the decoder's linear layers in a
+ * decode step (the reference's F.linear).  x (rows, k) bf16 with row stride
+ * x_row_stride elements, w (n, k) and out (rows, n) contiguous, all 16-byte
+ * aligned; products and sums in fp32, rounded once.  act 1: w is (2n, k), its
+ * first n rows the gate and its last n the up projection, and out =
+ * round(silu(gate) * up) on gate and up rounded to bf16 (what mkv_silu_mul
+ * gives on the product).  mkv_linear_supported says whether a product's sizes
+ * are taken (bf16, n a multiple of 16, k shared out evenly over 4, 8 or 16
+ * waves; not where the library is as fast); others return MKV_ERR_BAD_SHAPE,
+ * as do rows of x more than 2^20 elements apart. */
+int mkv_linear_supported(int64_t rows, int n, int k, int act, int dtype);
+int mkv_linear(void* out, const void* x, int64_t x_row_stride, const void* w, int64_t rows, int n,
+               int k, int act, int dtype, void* stream);
+
 /* ------------------------------------------------------------------------
  * Measurement helper (no counterpart in the reference; for benchmarks).
  *

@@ -1,0 +1,375 @@
+// The decoder's matrix products in a decode step: out = x W^T for up to 64
+// rows of x, with the SiLU-and-multiply of a gated MLP in the epilogue on
+// request.
+//
+// Reference: the engine's linear layers (linear.py: F.linear; the MLP's
+// activation.py:16-19), which a decode step calls with one row per sequence.
+// Operands are bf16, products and sums fp32 (v_mfma_f32_16x16x32_bf16),
+// rounded once.
+//
+// With so few rows a product is one pass over its weights (8 MB, the q/k/v of
+// a 1024-wide layer, are 1.3 us at 6.4 TB/s) and what costs is the latency
+// around it and the reads of x by every CU.  So k is shared out over the
+// waves of a workgroup until a wave's share is one memory round trip, and
+// there are about as many workgroups as CUs.  60 rows, weights not in cache,
+// us a product, before (the library's products, the gated one with
+// mkv_silu_mul behind it) and now: 4096 x 1024 11.3 / 6.2, 1024 x 2048 8.0 /
+// 5.2, 1024 x 3072 12.0 / 7.4, 2 x 3072 x 1024 gated 14.7 / 9.3, 151936 x 1024
+// 83 / 78; one row: 7.5 / 4.4, 8.4 / 4.9, 11.8 / 6.4, 10.4 / 5.6.
+//
+// The MFMA's rows are 16 output features (A = W, straight from memory: the
+// loads of two k-steps cover 16 whole lines), its columns 16 rows of x, so a
+// lane ends with 4 consecutive features of one row.
+#include "mkv_device.hpp"
+
+namespace mkv {
+namespace {
+
+constexpr int kLinMaxRows = 64;
+constexpr int64_t kLinMaxStride = (int64_t)1 << 20;  // x's offsets are 32 bits
+constexpr int kCus = 256;
+constexpr int kXcds = 8;
+
+struct LinearArgs {
+  uint16_t* out;      // (rows, n)
+  const uint16_t* x;  // (rows, k), row stride x_stride
+  const uint16_t* w;  // (n, k), with act: (2 n, k), gate rows then up rows
+  int64_t x_stride;
+  int rows, n, k;
+  int m_groups;       // groups of 16 MT rows
+};
+
+MKV_DEV bf16x8 ld_op(const uint16_t* p) { return __builtin_bit_cast(bf16x8, ld16(p)); }
+
+MKV_DEV uint2 pack_bf16x4(const float* x) {
+  return make_uint2(f32_to_bf16_bits(x[0]) | (f32_to_bf16_bits(x[1]) << 16),
+                    f32_to_bf16_bits(x[2]) | (f32_to_bf16_bits(x[3]) << 16));
+}
+
+// Element offset of k-step u from a lane's first (16 kg): the lane's 8
+// elements of two successive steps are 32 bytes together, so both steps' loads
+// touch the same 16 whole lines (the order within k is free).
+MKV_DEV constexpr int step_off(int u) { return 64 * (u >> 1) + 8 * (u & 1); }
+
+// Workgroup barrier that leaves loads in flight alone: this wave's LDS
+// accesses are done.
+MKV_DEV void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// ---------------------------------------------------------------------------
+// Split form: a workgroup owns 16 features (with ACT: 16 gate and the 16 up
+// features of the same outputs) and MT tiles of 16 rows, its waves share out
+// k, and their sums are joined in LDS (in wave order: the result does not
+// depend on timing).  A wave issues BLK k-steps' loads at once, so that a
+// product whose k is 32 BLK x waves is a single memory round trip.  x comes by
+// LDS DMA, whole lines an instruction: read as MFMA operands straight from
+// memory (16 half lines an instruction, the same ones by every CU) it took
+// 7.5 us for 4096 x 1024 at 60 rows, not 6.2.
+// ---------------------------------------------------------------------------
+template <int MT, int BLK, bool ACT>
+__global__ __launch_bounds__(1024) void linear_split_kernel(LinearArgs a) {
+  constexpr int NT = ACT ? 2 : 1;
+  extern __shared__ __align__(16) char smem[];
+  f32x4* part = reinterpret_cast<f32x4*>(smem);  // [wave][NT][MT][lane]
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int waves = blockDim.x >> 6;
+  const int c = lane & 15, kg = lane >> 4;
+  // consecutive workgroups (the row groups of one feature tile) on one XCD
+  const int nwg = gridDim.x;
+  const int b = nwg % kXcds == 0 ? (blockIdx.x % kXcds) * (nwg / kXcds) + blockIdx.x / kXcds : blockIdx.x;
+  const int n0 = (b / a.m_groups) * 16, m0 = (b % a.m_groups) * 16 * MT;
+
+  const int steps = a.k / 32 / waves;
+  const int kw = wave * steps * 32;
+  const uint16_t* wp[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) wp[t] = a.w + (int64_t)(n0 + t * a.n + c) * a.k + kw + 16 * kg;
+  // x by LDS DMA: BLK steps are kCh 16-byte chunks of each of 16 MT rows, slot
+  // i of the wave's part holding chunk (i % kCh) ^ swz of row i / kCh, so that
+  // a load instruction covers whole lines and the 16 rows of an operand read
+  // hit 16 positions of 256 bytes
+  constexpr int kCh = 4 * BLK, kRowsX = 16 * MT, kDmas = kRowsX * kCh / 64;
+  auto swz = [](int row) { return kCh % 16 == 0 ? row & 15 : (row >> 1) & 7; };
+  char* xs = smem + wave * (kRowsX * kCh * 16);
+  const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)a.x, (short)0, (int)(2 * ((a.rows - 1) * (int)a.x_stride + a.k)), 0x00020000);
+  uint32_t x_off[kDmas];
+#pragma unroll
+  for (int d = 0; d < kDmas; ++d) {
+    const int i = 64 * d + lane, row = i / kCh, ch = (i % kCh) ^ swz(row);
+    x_off[d] = 2u * (uint32_t)(min(m0 + row, a.rows - 1) * (int)a.x_stride + kw + 8 * ch);
+  }
+
+  f32x4 acc[NT][MT];
+#pragma unroll
+  for (int i = 0; i < NT; ++i)
+#pragma unroll
+    for (int j = 0; j < MT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int s = 0; s < steps; s += BLK) {
+    bf16x8 wf[BLK][NT];
+#pragma unroll
+    for (int d = 0; d < kDmas; ++d)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (__attribute__((address_space(3))) void*)(xs + 1024 * d), 16,
+                                               (int)x_off[d], 64 * s, 0, 0);
+#pragma unroll
+    for (int u = 0; u < BLK; ++u)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) wf[u][t] = ld_op(wp[t] + 32 * s + step_off(u));
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): x has landed (the wave's own: no barrier)
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int u = 0; u < BLK; ++u)
+#pragma unroll
+      for (int j = 0; j < MT; ++j) {
+        // chunk of elements step_off(u) + 16 kg of row 16 j + c
+        const int row = 16 * j + c, ch = (8 * (u >> 1) + (u & 1) + 2 * kg) ^ swz(row);
+        const bf16x8 xf = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(xs + (row * kCh + ch) * 16));
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u][i], xf, acc[i][j], 0, 0, 0);
+      }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  }
+  __syncthreads();  // the sums take the place of x
+#pragma unroll
+  for (int i = 0; i < NT; ++i)
+#pragma unroll
+    for (int j = 0; j < MT; ++j) part[((wave * NT + i) * MT + j) * 64 + lane] = acc[i][j];
+  __syncthreads();
+  for (int j = wave; j < MT; j += waves) {
+    f32x4 sum[NT];
+#pragma unroll
+    for (int i = 0; i < NT; ++i) sum[i] = part[(i * MT + j) * 64 + lane];
+#pragma unroll 4
+    for (int w = 1; w < waves; ++w)
+#pragma unroll
+      for (int i = 0; i < NT; ++i) {
+        const f32x4 p = part[((w * NT + i) * MT + j) * 64 + lane];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sum[i][r] += p[r];
+      }
+    const int m = m0 + 16 * j + c;
+    if (m >= a.rows) continue;
+    float y[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      if constexpr (ACT) {  // on gate and up rounded to bf16, as mkv_silu_mul reads them
+        const float g = bf16_bits_to_f32(f32_to_bf16_bits(sum[0][r]));
+        const float u = bf16_bits_to_f32(f32_to_bf16_bits(sum[NT - 1][r]));
+        y[r] = g / (1.0f + __expf(-g)) * u;
+      } else {
+        y[r] = sum[0][r];
+      }
+    }
+    *reinterpret_cast<uint2*>(a.out + (int64_t)m * a.n + n0 + 4 * kg) = pack_bf16x4(y);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Streaming form, for products with many more feature tiles than CUs (an LM
+// head): one 8-wave workgroup a CU takes a contiguous range of feature tiles.
+// Each wave keeps its eighth of x (4 k-steps of every row) in registers and
+// streams its eighth of the tiles' weights through a ring of three pairs of
+// tiles, two pairs (128 KB a CU) in flight ahead of the one it multiplies; the
+// waves' sums of a pair meet in LDS (double-buffered, one barrier a pair that
+// leaves the loads in flight), where wave w joins tile w / 4, rows 16 (w % 4).
+// 311 MB of weights: 63 us for one row, 78 for 60 (the writes of 18 MB of
+// logits); plain loads, since non-temporal ones took 68 and 88.
+// ---------------------------------------------------------------------------
+constexpr int kStreamWaves = 8;
+constexpr int kStreamSteps = 4;                              // k-steps of a wave
+constexpr int kStreamK = 32 * kStreamSteps * kStreamWaves;  // 1024
+
+template <int MT>
+__global__ __launch_bounds__(kStreamWaves* kWave) __attribute__((amdgpu_waves_per_eu(2))) void linear_stream_kernel(
+    LinearArgs a) {
+  extern __shared__ __align__(16) char smem[];
+  f32x4* part = reinterpret_cast<f32x4*>(smem);  // [2][wave][tile][MT][lane]
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = lane & 15, kg = lane >> 4;
+  const int tiles = a.n / 16;
+  const int nwg = gridDim.x;
+  const int b = nwg % kXcds == 0 ? (blockIdx.x % kXcds) * (nwg / kXcds) + blockIdx.x / kXcds : blockIdx.x;
+  const int t0 = (int)((int64_t)tiles * b / nwg), t1 = (int)((int64_t)tiles * (b + 1) / nwg);
+  const int pairs = (t1 - t0 + 1) / 2;
+  if (pairs == 0) return;
+
+  const int k0 = wave * 32 * kStreamSteps + 16 * kg;
+  const __amdgpu_buffer_rsrc_t wr =
+      __builtin_amdgcn_make_buffer_rsrc((void*)a.w, (short)0, (int)(2u * (uint32_t)a.n * kStreamK), 0x00020000);
+  const int w_off = 2 * (c * kStreamK + k0);
+  // (past the last tile: its weights again, so that every path issues the same
+  // loads and the waits count them exactly)
+  auto load_pair = [&](int p, bf16x8 (&f)[2][kStreamSteps]) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int tile_off = (int)(min(t0 + 2 * p + i, t1 - 1) * (2u * 16 * kStreamK));
+#pragma unroll
+      for (int u = 0; u < kStreamSteps; ++u)
+        f[i][u] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(wr, w_off + 2 * step_off(u), tile_off, 0));
+    }
+  };
+  bf16x8 f0[2][kStreamSteps], f1[2][kStreamSteps], f2[2][kStreamSteps], xf[MT][kStreamSteps];
+  load_pair(0, f0);
+#pragma unroll
+  for (int j = 0; j < MT; ++j)
+#pragma unroll
+    for (int u = 0; u < kStreamSteps; ++u)
+      xf[j][u] = ld_op(a.x + (int64_t)min(16 * j + c, a.rows - 1) * a.x_stride + k0 + step_off(u));
+  load_pair(1, f1);
+
+  const __amdgpu_buffer_rsrc_t out =
+      __builtin_amdgcn_make_buffer_rsrc(a.out, (short)0, (int)(2u * (uint32_t)a.rows * (uint32_t)a.n), 0x00020000);
+  const int red_tile = wave >> 2, red_m = 16 * (wave & 3) + c;
+  auto step = [&](int p, bf16x8 (&cur)[2][kStreamSteps], bf16x8 (&ahead)[2][kStreamSteps]) {
+    load_pair(p + 2, ahead);
+    __builtin_amdgcn_sched_barrier(0);
+    f32x4* buf = part + (p & 1) * (kStreamWaves * 2 * MT * 64);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      f32x4 acc[MT];
+#pragma unroll
+      for (int j = 0; j < MT; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int u = 0; u < kStreamSteps; ++u)
+#pragma unroll
+        for (int j = 0; j < MT; ++j)
+          acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur[i][u], xf[j][u], acc[j], 0, 0, 0);
+#pragma unroll
+      for (int j = 0; j < MT; ++j) buf[((wave * 2 + i) * MT + j) * 64 + lane] = acc[j];
+    }
+    lds_barrier();
+    f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < kStreamWaves; ++w) {
+      const f32x4 q = buf[((w * 2 + red_tile) * MT + min(wave & 3, MT - 1)) * 64 + lane];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sum[r] += q[r];
+    }
+    const float y[4] = {sum[0], sum[1], sum[2], sum[3]};
+    const uint2 o = pack_bf16x4(y);
+    const int tile = t0 + 2 * p + red_tile;
+    const bool ok = red_m < a.rows && tile < t1;
+    const uint32_t off = ok ? 2u * ((uint32_t)red_m * (uint32_t)a.n + (uint32_t)(tile * 16 + 4 * kg)) : 0xfffffff8u;
+    __builtin_amdgcn_raw_buffer_store_b64(u32x2{o.x, o.y}, out, (int)off, 0, 0);
+  };
+  for (int p = 0;;) {
+    step(p, f0, f2);
+    if (++p >= pairs) break;
+    step(p, f1, f0);
+    if (++p >= pairs) break;
+    step(p, f2, f1);
+    if (++p >= pairs) break;
+  }
+}
+
+// How a product runs; kind 0: not at all (the caller's own product).
+struct LinearPlan {
+  int kind;  // 1 split, 2 streaming
+  int mt, waves, blk;
+};
+
+LinearPlan plan_linear(int64_t rows, int n, int k, int act) {
+  LinearPlan p{0, 0, 0, 0};
+  if (rows < 1 || rows > kLinMaxRows || n < 16 || n % 16 || k < 32 || k % 32) return p;
+  const int m_tiles = (int)(rows + 15) / 16, n_tiles = n / 16;
+  // Streaming from 8 feature tiles a CU on (its offsets are 32 bits), for more
+  // than 16 rows: at most 16 are as fast or faster in the library (151936 x
+  // 1024: one row 62 us and 63 here, 16 rows 65 and 69, 17 rows 75 and 70).
+  if (!act && n_tiles >= 8 * kCus) {
+    if (k != kStreamK || m_tiles < 2 || (int64_t)k * n * 2 >= ((int64_t)1 << 31)) return p;
+    p.kind = 2;
+    p.mt = m_tiles;
+    return p;
+  }
+  // Split up to 2^20 (feature tiles x row tiles x k: 32 MB of x read by the
+  // workgroups) and k 4096; past either the library is as fast or faster.
+  // 64 rows: 4096 x 1024 11.6 us and 7.7 here, 2048 x 2048 11.9 / 7.2, 6144 x
+  // 1024 11.9 / 12.2, 4096 x 4096 15.4 / 21.0; 16 rows: 4096 x 4096 15.9 /
+  // 11.2, 6144 x 4096 16.0 / 17.2, 2048 x 6144 12.2 / 13.1.
+  if ((int64_t)n_tiles * m_tiles * k > (1 << 20) || k > 4096) return p;
+  // Waves: as many as leave each of them one or two times 4 or 6 k-steps
+  // (2560 = 4 waves x 5 times 4 at 32 rows: 9.5 us and 10.5 here).
+  const int steps = k / 32;
+  for (int waves : {16, 8, 4}) {
+    if (steps % waves) continue;
+    const int per = steps / waves;
+    if (waves == 16 && per < 4) continue;
+    const int blk = per % 4 == 0 ? 4 : (per % 6 == 0 ? 6 : 0);
+    if (!blk || per > 2 * blk) continue;
+    p.waves = waves;
+    p.blk = blk;
+    break;
+  }
+  if (!p.blk) return p;
+  p.kind = 1;
+  // Rows a workgroup: all of them (the weights are read once) where that still
+  // makes a workgroup a CU, else fewer: 1024 features are 64 tiles, 256
+  // workgroups at 16 rows each.
+  for (p.mt = m_tiles > 2 ? 4 : m_tiles; p.mt > 1 && (int64_t)n_tiles * ((m_tiles + p.mt - 1) / p.mt) < kCus;) p.mt /= 2;
+  if (act && p.mt == 4) p.mt = 2;
+  if ((p.waves == 16 || p.blk == 6) && p.mt == 4) p.mt = 2;
+  return p;
+}
+
+template <int MT, bool ACT>
+void launch_split(const LinearArgs& a, const LinearPlan& p, hipStream_t s) {
+  const dim3 grid((unsigned)(a.n / 16 * a.m_groups)), block(p.waves * kWave);
+  const size_t sums = (size_t)p.waves * (ACT ? 2 : 1) * MT * 1024, x = (size_t)p.waves * 16 * MT * p.blk * 64;
+  const size_t lds = sums > x ? sums : x;
+  if (MT == 4 || p.blk == 4)
+    hipLaunchKernelGGL((linear_split_kernel<MT, 4, ACT>), grid, block, lds, s, a);
+  else
+    hipLaunchKernelGGL((linear_split_kernel<MT, MT == 4 ? 4 : 6, ACT>), grid, block, lds, s, a);
+}
+
+template <int MT>
+void launch_stream(const LinearArgs& a, hipStream_t s) {
+  const size_t lds = (size_t)2 * kStreamWaves * 2 * MT * 64 * sizeof(f32x4);
+  hipLaunchKernelGGL(linear_stream_kernel<MT>, dim3(kCus), dim3(kStreamWaves * kWave), lds, s, a);
+}
+
+}  // namespace
+}  // namespace mkv
+
+using namespace mkv;
+
+extern "C" int mkv_linear_supported(int64_t rows, int n, int k, int act, int dtype) {
+  return dtype == MKV_DTYPE_BF16 && plan_linear(rows, n, k, act).kind != 0;
+}
+
+extern "C" int mkv_linear(void* out, const void* x, int64_t x_row_stride, const void* w, int64_t rows, int n,
+                          int k, int act, int dtype, void* stream) {
+  if (dtype != MKV_DTYPE_BF16) return MKV_ERR_UNSUPPORTED_DTYPE;
+  const LinearPlan p = plan_linear(rows, n, k, act);
+  if (!p.kind || x_row_stride < k || x_row_stride > kLinMaxStride) return MKV_ERR_BAD_SHAPE;
+  if (!out || !x || !w) return MKV_ERR_NULL_POINTER;
+  if (((reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 15u) ||
+      x_row_stride % 8)
+    return MKV_ERR_MISALIGNED;
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  LinearArgs a{reinterpret_cast<uint16_t*>(out), reinterpret_cast<const uint16_t*>(x),
+               reinterpret_cast<const uint16_t*>(w), x_row_stride, (int)rows, n, k, 1};
+  const int m_tiles = (int)(rows + 15) / 16;
+  if (p.kind == 2) {
+    switch (p.mt) {
+      case 2: launch_stream<2>(a, s); break;
+      case 3: launch_stream<3>(a, s); break;
+      default: launch_stream<4>(a, s); break;
+    }
+  } else {
+    a.m_groups = (m_tiles + p.mt - 1) / p.mt;
+    if (act) {
+      if (p.mt == 2) launch_split<2, true>(a, p, s);
+      else launch_split<1, true>(a, p, s);
+    } else {
+      if (p.mt == 4) launch_split<4, false>(a, p, s);
+      else if (p.mt == 2) launch_split<2, false>(a, p, s);
+      else launch_split<1, false>(a, p, s);
+    }
+  }
+  return (int)hipGetLastError();
+}

@@ -15,8 +15,9 @@ tokens per second; it is not a port of the reference's runner.  The pieces:
   handed out as the tokens that need them are scheduled; a running sequence
   that cannot get a block preempts the newest running sequence, which
   starts again from its prompt (recompute).
-* :class:`Qwen3Model`: the Qwen3 decoder (qwen3.py:73-284) in bf16 on torch
-  GEMMs, with the attention layer's producer fused
+* :class:`Qwen3Model`: the Qwen3 decoder (qwen3.py:73-284) in bf16, its
+  products on mkv_linear for the few rows of a decode step and on torch
+  otherwise, with the attention layer's producer fused
   (:func:`mkv.producer.qkv_norm_rope_append`: q/k RMSNorm + RoPE + the FP8
   append) and :class:`mkv.Attention` for the paged attention; embeddings tied
   to the LM head.
@@ -260,6 +261,38 @@ def silu_and_mul(x: torch.Tensor) -> torch.Tensor:
     return out
 
 
+def _own_product(x: torch.Tensor, w: torch.Tensor, n: int, act: int) -> bool:
+    """Whether mkv_linear takes x w^T: a few bf16 rows on the GPU with no
+    gradient to record, in sizes it shares out evenly."""
+    return (x.is_cuda and x.dtype == w.dtype == torch.bfloat16 and x.dim() == w.dim() == 2
+            and x.device == w.device and x.shape[1] == w.shape[1] and 0 < x.shape[0] <= 64
+            and x.stride(1) == 1 and x.shape[1] <= x.stride(0) <= 1 << 20 and x.stride(0) % 8 == 0
+            and w.is_contiguous()
+            and (x.data_ptr() | w.data_ptr()) % 16 == 0
+            and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))
+            and bool(_lib.query("mkv_linear_supported", x.shape[0], n, x.shape[1], act, _dtype_code(x, "x"))))
+
+
+def _product(x: torch.Tensor, w: torch.Tensor, n: int, act: int) -> torch.Tensor:
+    out = torch.empty(x.shape[0], n, dtype=x.dtype, device=x.device)
+    _lib.call("mkv_linear", out.data_ptr(), x.data_ptr(), x.stride(0), w.data_ptr(), x.shape[0], n,
+              x.shape[1], act, _dtype_code(x, "x"), _stream(x.device))
+    return out
+
+
+def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """x w^T: for the few rows of a decode step one pass over the weights
+    (mkv_linear), else torch's product."""
+    return _product(x, w, w.shape[0], 0) if _own_product(x, w, w.shape[0], 0) else F.linear(x, w)
+
+
+def gated_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """silu(x gate^T) * (x up^T), w = [gate; up]: in a decode step one kernel
+    with the activation in its epilogue."""
+    inter = w.shape[0] // 2
+    return _product(x, w, inter, 1) if _own_product(x, w, inter, 1) else silu_and_mul(F.linear(x, w))
+
+
 class Qwen3Model(torch.nn.Module):
     """Random-init Qwen3 decoder (weights N(0, std), norm weights 1) whose
     attention layers run on the mkv operators.  A decode step runs each
@@ -360,7 +393,7 @@ class Qwen3Model(torch.nn.Module):
                 h = rms_norm(x, lay["in_norm"], cfg.eps)
             else:
                 h = rms_norm(x, lay["in_norm"], cfg.eps, residual)
-            qkv = F.linear(h, lay["qkv"])
+            qkv = linear(h, lay["qkv"])
             att = lay["attn"]
             ctx = C.current_context()
             if self.fuse_decode_step and not ctx.is_prefill:
@@ -379,13 +412,13 @@ class Qwen3Model(torch.nn.Module):
                     eps=cfg.eps, kv_cache_dtype=att.kv_cache_dtype, k_scale=att.k_scale,
                     v_scale=att.v_scale, return_k=full_prefill)
                 o = self.attention(li, q, k, v)
-            x = F.linear(o, lay["o"])
+            x = linear(o, lay["o"])
             h = rms_norm(x, lay["post_norm"], cfg.eps, residual)
-            x = F.linear(silu_and_mul(F.linear(h, lay["gate_up"])), lay["down"])
+            x = linear(gated_linear(h, lay["gate_up"]), lay["down"])
         return rms_norm(x, self.final_norm, cfg.eps, residual)
 
     def logits(self, hidden: torch.Tensor) -> torch.Tensor:
-        return F.linear(hidden, self.embed)
+        return linear(hidden, self.embed)
 
 
 def sample(logits: torch.Tensor, temperature: torch.Tensor, gen: torch.Generator) -> torch.Tensor:

@@ -12,6 +12,7 @@ import pytest
 import torch
 
 from conftest import announce
+from mkv import _lib
 from mkv import engine as E
 
 pytestmark = pytest.mark.gpu
@@ -69,3 +70,66 @@ def test_silu_mul_strided_rows(dev):
     out = E.silu_and_mul(x)
     a, b = x[:, :64].double().cpu(), x[:, 64:].double().cpu()
     _check(out, a / (1 + torch.exp(-a)) * b, torch.bfloat16)
+
+
+def _ulp(x):
+    return torch.exp2(torch.floor(torch.log2(x.abs().clamp(min=2.0 ** -126))) - 7)  # bf16
+
+
+@pytest.mark.parametrize("rows", [1, 15, 16, 17, 33, 60, 64])
+@pytest.mark.parametrize("n,k", [(16, 512), (48, 768), (4096, 1024), (1024, 2048), (112, 3072), (80, 4096), (48, 1536), (32816, 1024)])
+@pytest.mark.parametrize("strided", [False, True])
+def test_linear(dev, rows, n, k, strided):
+    """mkv_linear in every form (4, 8 and 16 waves, 4 and 6 k-steps, one or
+    two loads of k, 16 to 64 rows a workgroup, streaming), with rows and
+    feature tiles that do not fill them.  Bound: half an ulp of the output
+    and k fp32 roundings of the sum of |x| |w|."""
+    announce(f"linear {rows} x {n} x {k} strided={strided}")
+    assert _lib.query("mkv_linear_supported", rows, n, k, 0, _lib.DTYPE_BF16) == (n < 32768 or rows > 16)
+    g = torch.Generator().manual_seed(rows * 7 + n)
+    w = torch.randn(n, k, generator=g).bfloat16().to(dev)
+    x = torch.randn(rows, k + 8, generator=g).bfloat16().to(dev)
+    x = x[:, :k] if strided else x[:, :k].contiguous()
+    got = E.linear(x, w).double()
+    want, mag = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    assert bool(((got - want).abs() <= 0.5 * _ulp(want) + k * 2.0 ** -24 * mag).all())
+
+
+@pytest.mark.parametrize("rows", [1, 17, 60])
+@pytest.mark.parametrize("inter,k", [(16, 512), (3072, 1024), (48, 3072)])
+def test_gated_linear(dev, rows, inter, k):
+    """The gated product against silu(gate) * up in 64 bits.  Bound: gate and
+    up are rounded to bf16 (half an ulp each, silu's slope at most 1.1) and
+    so is the result, plus the products' fp32 sums."""
+    announce(f"gated linear {rows} x {inter} x {k}")
+    assert _lib.query("mkv_linear_supported", rows, inter, k, 1, _lib.DTYPE_BF16)
+    g = torch.Generator().manual_seed(rows + inter)
+    w = (torch.randn(2 * inter, k, generator=g) * 2 / k ** 0.5).bfloat16().to(dev)
+    x = torch.randn(rows, k, generator=g).bfloat16().to(dev)
+    got = E.gated_linear(x, w).double()
+    p, mag = x.double() @ w.double().t(), k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+    e = 0.5 * _ulp(p) * 1.01 + mag
+    gate, up = p.chunk(2, -1)
+    eg, eu = e.chunk(2, -1)
+    silu = torch.nn.functional.silu(gate)
+    want = silu * up
+    bound = 1.1 * eg * (up.abs() + eu) + silu.abs() * eu + 0.5 * _ulp(want) * 1.01 + 1e-6 * want.abs()
+    assert bool(((got - want).abs() <= bound).all())
+
+
+def test_linear_leaves_other_products_to_torch(dev):
+    """Sizes, types and layouts that mkv_linear does not take give torch's
+    product: many rows, fp16, a transposed weight, a gradient to record."""
+    g = torch.Generator().manual_seed(3)
+    w = torch.randn(64, 1024, generator=g).to(dev)
+    x = torch.randn(65, 1024, generator=g).to(dev)
+    wb, xb = w.bfloat16(), x.bfloat16()
+    wt = w.t().contiguous().bfloat16().t()
+    assert not any(_lib.query("mkv_linear_supported", m, n, k, 0, _lib.DTYPE_BF16)
+                   for m, n, k in ((65, 64, 1024), (64, 6144, 1024), (16, 2048, 6144), (8, 2560, 2560),
+                                   (1, 24, 1024), (1, 16, 16), (0, 16, 1024)))
+    for a, b in ((xb, wb), (x[:8].half(), w.half()), (x[:8], w), (xb[:8], wt), (xb[:8, :40], wb[:, :40].contiguous())):
+        assert torch.equal(E.linear(a, b), torch.nn.functional.linear(a, b))
+    wr = wb.clone().requires_grad_(True)
+    E.linear(xb[:8], wr).float().sum().backward()
+    assert wr.grad is not None
