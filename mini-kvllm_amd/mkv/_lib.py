@@ -130,15 +130,24 @@ def load(path: str | Path | None = None) -> ctypes.CDLL:
         return lib
 
 
+# Bound entry points of the library that load() keeps, so that a launch costs
+# no lock and no attribute lookup.
+_entries: dict[str, ctypes._CFuncPtr] = {}
+
+
+def _entry(name: str):
+    fn = _entries[name] = getattr(load(), name)
+    return fn
+
+
 def call(name: str, *args) -> None:
     """Invoke an int-returning entry point and raise MkvError on failure."""
-    lib = load()
-    status = getattr(lib, name)(*args)
+    status = (_entries.get(name) or _entry(name))(*args)
     if status != 0:
-        msg = lib.mkv_status_string(status).decode()
+        msg = load().mkv_status_string(status).decode()
         raise MkvError(name, status, msg)
 
 
 def query(name: str, *args):
     """Invoke a size/info entry point and return its value."""
-    return getattr(load(), name)(*args)
+    return (_entries.get(name) or _entry(name))(*args)

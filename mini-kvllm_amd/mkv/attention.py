@@ -49,6 +49,8 @@ _DTYPES = {
     torch.int8: _lib.DTYPE_I8,
 }
 
+_QUANT_CODES = (_lib.DTYPE_FP8E4M3, _lib.DTYPE_I8)
+
 # kv_cache_dtype strings of the reference's quantised modes and the scale
 # granularity each uses (model_runner.py:222-229, :324-338).
 PER_TOKEN_HEAD_MODES = ("fp8_per_token_head", "int8_per_token_head")
@@ -70,7 +72,10 @@ def _dtype_code(t: torch.Tensor, what: str) -> int:
 
 def _require_gpu(*tensors: torch.Tensor) -> torch.device:
     dev = tensors[0].device
+    idx = dev.index
     for t in tensors:
+        if t.is_cuda and t.get_device() == idx:  # (no device object per tensor)
+            continue
         if t.device.type != "cuda":
             raise ValueError("mkv kernels run on the GPU only; got a tensor on "
                              f"{t.device} (there is no CPU fallback)")
@@ -80,7 +85,10 @@ def _require_gpu(*tensors: torch.Tensor) -> torch.device:
 
 
 def _stream(dev: torch.device) -> int:
-    return torch.cuda.current_stream(dev).cuda_stream
+    """The raw handle of the device's current stream (without the Stream
+    object that torch.cuda.current_stream builds)."""
+    return torch._C._cuda_getCurrentRawStream(
+        dev.index if dev.index is not None else torch.cuda.current_device())
 
 
 _side_streams: dict[int, torch.cuda.Stream] = {}
@@ -115,8 +123,8 @@ def _token_rows(x: torch.Tensor) -> torch.Tensor:
     """(tokens, kv_heads, head_dim) with contiguous rows; a row stride larger
     than the row (e.g. a k/v view into a fused qkv buffer) is kept as is."""
     T, H, D = x.shape
-    if x.stride(2) == 1 and x.stride(1) == D and x.stride(0) >= H * D and \
-            (x.stride(0) * x.element_size()) % 16 == 0 and x.data_ptr() % 16 == 0:
+    s0, s1, s2 = x.stride()
+    if s2 == 1 and s1 == D and s0 >= H * D and (s0 * x.element_size()) % 16 == 0 and x.data_ptr() % 16 == 0:
         return x
     return x.contiguous()
 
@@ -162,10 +170,11 @@ def _one_dtype(key: torch.Tensor, value: torch.Tensor):
 def _check_cache(k_cache: torch.Tensor, v_cache: torch.Tensor, num_kv_heads: int, head_dim: int):
     if k_cache.dtype != v_cache.dtype:
         raise TypeError(f"k_cache and v_cache must share a dtype; got {k_cache.dtype} and {v_cache.dtype}")
-    if k_cache.dim() != 4 or k_cache.shape != v_cache.shape:
+    shape = k_cache.shape
+    if len(shape) != 4 or shape != v_cache.shape:
         raise ValueError("k_cache/v_cache must both be (num_blocks, block_size, num_kv_heads, "
                          f"head_dim); got {tuple(k_cache.shape)} and {tuple(v_cache.shape)}")
-    if k_cache.shape[2] != num_kv_heads or k_cache.shape[3] != head_dim:
+    if shape[2] != num_kv_heads or shape[3] != head_dim:
         raise ValueError(f"cache head layout {tuple(k_cache.shape[2:])} != ({num_kv_heads}, {head_dim})")
     if not (k_cache.is_contiguous() and v_cache.is_contiguous()):
         raise ValueError("k_cache/v_cache must be contiguous per layer")
@@ -348,8 +357,9 @@ def _decode(query, k_cache, v_cache, block_tables, context_lens, scale, num_head
             out=None, per_token_head=False) -> torch.Tensor:
     dev = _require_gpu(query, k_cache, v_cache, block_tables, context_lens)
     query = query.contiguous()
-    batch = query.shape[0]
-    if query.dim() != 3 or query.shape[1] != num_heads or query.shape[2] != head_dim:
+    q_shape = query.shape
+    batch = q_shape[0]
+    if len(q_shape) != 3 or q_shape[1] != num_heads or q_shape[2] != head_dim:
         raise ValueError(f"query must be (batch, {num_heads}, {head_dim}); got {tuple(query.shape)}")
     _check_cache(k_cache, v_cache, num_kv_heads, head_dim)
     if out is None:
@@ -358,23 +368,24 @@ def _decode(query, k_cache, v_cache, block_tables, context_lens, scale, num_head
         return out
     bt = _block_table(block_tables)
     cl = _ctx_lens(context_lens)
-    if bt.dim() != 2 or bt.shape[0] < batch or cl.numel() < batch:
+    bt_shape = bt.shape
+    if len(bt_shape) != 2 or bt_shape[0] < batch or cl.numel() < batch:
         raise ValueError(f"block_tables {tuple(bt.shape)} / context_lens {tuple(cl.shape)} cover fewer "
                          f"than the batch's {batch} sequences")
-    max_blocks = bt.shape[1]
-    bs = k_cache.shape[1]
-    quant = k_cache.dtype in (torch.float8_e4m3fn, torch.int8)
+    max_blocks = bt_shape[1]
+    num_blocks, bs = k_cache.shape[:2]
+    kv_code = _dtype_code(k_cache, "k_cache")
+    quant = kv_code in _QUANT_CODES
     if quant and (k_scale is None or v_scale is None):
         raise ValueError("a quantised cache needs k_scale and v_scale")
     if per_token_head:
         _check_token_scales(k_scale, v_scale, k_cache)
     nbytes = _lib.query("mkv_paged_decode_workspace_size", batch, num_heads, num_kv_heads,
-                        max_blocks, bs, head_dim, _dtype_code(k_cache, "k_cache"), split_tokens)
+                        max_blocks, bs, head_dim, kv_code, split_tokens)
     ws = _workspace(dev, "decode", nbytes) if nbytes else None
     _lib.call(
         "mkv_paged_decode", out.data_ptr(), out.stride(0), query.data_ptr(), query.stride(0),
-        _dtype_code(query, "query"), k_cache.data_ptr(), v_cache.data_ptr(),
-        _dtype_code(k_cache, "k_cache"), k_cache.shape[0],
+        _dtype_code(query, "query"), k_cache.data_ptr(), v_cache.data_ptr(), kv_code, num_blocks,
         k_scale.data_ptr() if quant else None, v_scale.data_ptr() if quant else None,
         _lib.SCALE_PER_TOKEN_HEAD if per_token_head else _lib.SCALE_PER_TENSOR,
         bt.data_ptr(), bt.stride(0), max_blocks, cl.data_ptr(), _index_dtype(cl), batch,
