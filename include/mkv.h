@@ -535,9 +535,13 @@ int mkv_silu_mul(void* out, const void* x, int64_t x_row_stride, int64_t rows,
  * gives on the product).  mkv_linear_supported says whether a product's sizes
  * are taken (bf16, n a multiple of 16, k shared out evenly over 4, 8 or 16
  * waves; not where the library is as fast); others return MKV_ERR_BAD_SHAPE,
- * as do rows of x more than 2^20 elements apart. */
-int mkv_linear_supported(int64_t rows, int n, int k, int act, int dtype);
-int mkv_linear(void* out, const void* x, int64_t x_row_stride, const void* w, int64_t rows, int n,
+ * as do rows of x more than 2^20 elements apart.  norm_weight (k,) non-NULL
+ * (norm 1 in the query): the product of the rows that mkv_rmsnorm makes of x
+ * without a residual.  residual (rows, n) non-NULL (act 0, fewer than 32768
+ * features; it may be out): out = round(round(product) + residual). */
+int mkv_linear_supported(int64_t rows, int n, int k, int act, int norm, int dtype);
+int mkv_linear(void* out, const void* x, int64_t x_row_stride, const void* w,
+               const void* norm_weight, float eps, const void* residual, int64_t rows, int n,
                int k, int act, int dtype, void* stream);
 
 /* ------------------------------------------------------------------------

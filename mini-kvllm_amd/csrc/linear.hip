@@ -37,6 +37,9 @@ struct LinearArgs {
   int64_t x_stride;
   int rows, n, k;
   int m_groups;       // groups of 16 MT rows
+  const uint16_t* norm;      // NORM: RMSNorm weight (k)
+  float eps;
+  const uint16_t* residual;  // (rows, n) added to the rounded product, or null; may be out
 };
 
 MKV_DEV bf16x8 ld_op(const uint16_t* p) { return __builtin_bit_cast(bf16x8, ld16(p)); }
@@ -69,7 +72,15 @@ MKV_DEV void lds_barrier() {
 // memory (16 half lines an instruction, the same ones by every CU) it took
 // 7.5 us for 4096 x 1024 at 60 rows, not 6.2.
 // ---------------------------------------------------------------------------
-template <int MT, int BLK, bool ACT>
+//
+// NORM (products of one round trip): x's rows are RMS-normalised on the way,
+// round(x * (1 / rms) * weight) as mkv_rmsnorm rounds it.  Every workgroup
+// works the rows' sums of squares out of the x it reads anyway, its waves'
+// parts joined in LDS ahead of the product.  At 60 rows the two norms of a
+// layer took 5 us each as launches of their own (add, norm, one row a wave);
+// with them and the residual additions here a decode step of 8 layers went
+// from 580 to 556 us.
+template <int MT, int BLK, bool ACT, bool NORM>
 __global__ __launch_bounds__(1024) void linear_split_kernel(LinearArgs a) {
   constexpr int NT = ACT ? 2 : 1;
   extern __shared__ __align__(16) char smem[];
@@ -109,7 +120,7 @@ __global__ __launch_bounds__(1024) void linear_split_kernel(LinearArgs a) {
 #pragma unroll
     for (int j = 0; j < MT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   for (int s = 0; s < steps; s += BLK) {
-    bf16x8 wf[BLK][NT];
+    bf16x8 wf[BLK][NT], nf[NORM ? BLK : 1];
 #pragma unroll
     for (int d = 0; d < kDmas; ++d)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (__attribute__((address_space(3))) void*)(xs + 1024 * d), 16,
@@ -118,15 +129,55 @@ __global__ __launch_bounds__(1024) void linear_split_kernel(LinearArgs a) {
     for (int u = 0; u < BLK; ++u)
 #pragma unroll
       for (int t = 0; t < NT; ++t) wf[u][t] = ld_op(wp[t] + 32 * s + step_off(u));
+    if constexpr (NORM) {
+#pragma unroll
+      for (int u = 0; u < BLK; ++u) nf[u] = ld_op(a.norm + kw + 16 * kg + 32 * s + step_off(u));
+    }
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): x has landed (the wave's own: no barrier)
     asm volatile("" ::: "memory");
+    auto x_op = [&](int u, int j) {  // chunk of elements step_off(u) + 16 kg of row 16 j + c
+      const int row = 16 * j + c, ch = (8 * (u >> 1) + (u & 1) + 2 * kg) ^ swz(row);
+      return __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(xs + (row * kCh + ch) * 16));
+    };
+    float inv[MT];
+    if constexpr (NORM) {
+      float* sq = reinterpret_cast<float*>(smem + waves * (kRowsX * kCh * 16));  // [MT][16][wave]
+#pragma unroll
+      for (int j = 0; j < MT; ++j) {
+        float ss = 0.0f;
+#pragma unroll
+        for (int u = 0; u < BLK; ++u) {
+          const bf16x8 xf = x_op(u, j);
+#pragma unroll
+          for (int e = 0; e < 8; e += 2) {
+            const bf16x2 p = {xf[e], xf[e + 1]};
+            ss = __builtin_amdgcn_fdot2_f32_bf16(p, p, ss, false);
+          }
+        }
+        ss += __shfl_xor(ss, 16);
+        ss += __shfl_xor(ss, 32);
+        if (kg == 0) sq[(16 * j + c) * waves + wave] = ss;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < MT; ++j) {
+        float ss = 0.0f;
+        for (int w = 0; w < waves; w += 4) {
+          const f32x4 q = *reinterpret_cast<const f32x4*>(sq + (16 * j + c) * waves + w);
+          ss += (q[0] + q[1]) + (q[2] + q[3]);
+        }
+        inv[j] = 1.0f / __builtin_sqrtf(ss / (float)a.k + a.eps);
+      }
+    }
 #pragma unroll
     for (int u = 0; u < BLK; ++u)
 #pragma unroll
       for (int j = 0; j < MT; ++j) {
-        // chunk of elements step_off(u) + 16 kg of row 16 j + c
-        const int row = 16 * j + c, ch = (8 * (u >> 1) + (u & 1) + 2 * kg) ^ swz(row);
-        const bf16x8 xf = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(xs + (row * kCh + ch) * 16));
+        bf16x8 xf = x_op(u, j);
+        if constexpr (NORM) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) xf[e] = (__bf16)((float)xf[e] * inv[j] * (float)nf[u][e]);
+        }
 #pragma unroll
         for (int i = 0; i < NT; ++i)
           acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u][i], xf, acc[i][j], 0, 0, 0);
@@ -153,6 +204,9 @@ __global__ __launch_bounds__(1024) void linear_split_kernel(LinearArgs a) {
       }
     const int m = m0 + 16 * j + c;
     if (m >= a.rows) continue;
+    const int64_t o = (int64_t)m * a.n + n0 + 4 * kg;
+    uint2 res = make_uint2(0, 0);
+    if (!ACT && a.residual) res = *reinterpret_cast<const uint2*>(a.residual + o);
     float y[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -162,9 +216,12 @@ __global__ __launch_bounds__(1024) void linear_split_kernel(LinearArgs a) {
         y[r] = g / (1.0f + __expf(-g)) * u;
       } else {
         y[r] = sum[0][r];
+        if (a.residual)  // the product rounded first, as a product of its own
+          y[r] = bf16_bits_to_f32(f32_to_bf16_bits(y[r])) +
+                 bf16_bits_to_f32(((r < 2 ? res.x : res.y) >> (16 * (r & 1))) & 0xffffu);
       }
     }
-    *reinterpret_cast<uint2*>(a.out + (int64_t)m * a.n + n0 + 4 * kg) = pack_bf16x4(y);
+    *reinterpret_cast<uint2*>(a.out + o) = pack_bf16x4(y);
   }
 }
 
@@ -272,7 +329,7 @@ struct LinearPlan {
   int mt, waves, blk;
 };
 
-LinearPlan plan_linear(int64_t rows, int n, int k, int act) {
+LinearPlan plan_linear(int64_t rows, int n, int k, int act, int norm) {
   LinearPlan p{0, 0, 0, 0};
   if (rows < 1 || rows > kLinMaxRows || n < 16 || n % 16 || k < 32 || k % 32) return p;
   const int m_tiles = (int)(rows + 15) / 16, n_tiles = n / 16;
@@ -280,7 +337,7 @@ LinearPlan plan_linear(int64_t rows, int n, int k, int act) {
   // than 16 rows: at most 16 are as fast or faster in the library (151936 x
   // 1024: one row 62 us and 63 here, 16 rows 65 and 69, 17 rows 75 and 70).
   if (!act && n_tiles >= 8 * kCus) {
-    if (k != kStreamK || m_tiles < 2 || (int64_t)k * n * 2 >= ((int64_t)1 << 31)) return p;
+    if (norm || k != kStreamK || m_tiles < 2 || (int64_t)k * n * 2 >= ((int64_t)1 << 31)) return p;
     p.kind = 2;
     p.mt = m_tiles;
     return p;
@@ -299,7 +356,7 @@ LinearPlan plan_linear(int64_t rows, int n, int k, int act) {
     const int per = steps / waves;
     if (waves == 16 && per < 4) continue;
     const int blk = per % 4 == 0 ? 4 : (per % 6 == 0 ? 6 : 0);
-    if (!blk || per > 2 * blk) continue;
+    if (!blk || per > (norm ? 1 : 2) * blk) continue;
     p.waves = waves;
     p.blk = blk;
     break;
@@ -312,18 +369,30 @@ LinearPlan plan_linear(int64_t rows, int n, int k, int act) {
   for (p.mt = m_tiles > 2 ? 4 : m_tiles; p.mt > 1 && (int64_t)n_tiles * ((m_tiles + p.mt - 1) / p.mt) < kCus;) p.mt /= 2;
   if (act && p.mt == 4) p.mt = 2;
   if ((p.waves == 16 || p.blk == 6) && p.mt == 4) p.mt = 2;
+  if (act && norm && p.blk == 6) p.mt = 1;  // (two row tiles do not fit the registers)
   return p;
 }
 
-template <int MT, bool ACT>
+template <int MT, bool ACT, bool NORM>
 void launch_split(const LinearArgs& a, const LinearPlan& p, hipStream_t s) {
   const dim3 grid((unsigned)(a.n / 16 * a.m_groups)), block(p.waves * kWave);
-  const size_t sums = (size_t)p.waves * (ACT ? 2 : 1) * MT * 1024, x = (size_t)p.waves * 16 * MT * p.blk * 64;
+  const size_t sums = (size_t)p.waves * (ACT ? 2 : 1) * MT * 1024;
+  const size_t x = (size_t)p.waves * MT * (16 * p.blk * 64 + (NORM ? 64 : 0));
   const size_t lds = sums > x ? sums : x;
-  if (MT == 4 || p.blk == 4)
-    hipLaunchKernelGGL((linear_split_kernel<MT, 4, ACT>), grid, block, lds, s, a);
+  constexpr bool kFour = MT == 4 || (MT == 2 && ACT && NORM);  // plan_linear's
+  if (kFour || p.blk == 4)
+    hipLaunchKernelGGL((linear_split_kernel<MT, 4, ACT, NORM>), grid, block, lds, s, a);
   else
-    hipLaunchKernelGGL((linear_split_kernel<MT, MT == 4 ? 4 : 6, ACT>), grid, block, lds, s, a);
+    hipLaunchKernelGGL((linear_split_kernel<MT, kFour ? 4 : 6, ACT, NORM>), grid, block, lds, s, a);
+}
+
+template <bool ACT, bool NORM>
+void launch_rows(const LinearArgs& a, const LinearPlan& p, hipStream_t s) {
+  if constexpr (!ACT) {
+    if (p.mt == 4) return launch_split<4, false, NORM>(a, p, s);
+  }
+  if (p.mt == 2) launch_split<2, ACT, NORM>(a, p, s);
+  else launch_split<1, ACT, NORM>(a, p, s);
 }
 
 template <int MT>
@@ -337,22 +406,26 @@ void launch_stream(const LinearArgs& a, hipStream_t s) {
 
 using namespace mkv;
 
-extern "C" int mkv_linear_supported(int64_t rows, int n, int k, int act, int dtype) {
-  return dtype == MKV_DTYPE_BF16 && plan_linear(rows, n, k, act).kind != 0;
+extern "C" int mkv_linear_supported(int64_t rows, int n, int k, int act, int norm, int dtype) {
+  return dtype == MKV_DTYPE_BF16 && plan_linear(rows, n, k, act, norm).kind != 0;
 }
 
-extern "C" int mkv_linear(void* out, const void* x, int64_t x_row_stride, const void* w, int64_t rows, int n,
-                          int k, int act, int dtype, void* stream) {
+extern "C" int mkv_linear(void* out, const void* x, int64_t x_row_stride, const void* w,
+                          const void* norm_weight, float eps, const void* residual, int64_t rows, int n, int k,
+                          int act, int dtype, void* stream) {
   if (dtype != MKV_DTYPE_BF16) return MKV_ERR_UNSUPPORTED_DTYPE;
-  const LinearPlan p = plan_linear(rows, n, k, act);
+  const LinearPlan p = plan_linear(rows, n, k, act, norm_weight != nullptr);
   if (!p.kind || x_row_stride < k || x_row_stride > kLinMaxStride) return MKV_ERR_BAD_SHAPE;
+  if (residual && (act || p.kind == 2)) return MKV_ERR_BAD_SHAPE;
   if (!out || !x || !w) return MKV_ERR_NULL_POINTER;
-  if (((reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 15u) ||
+  if (((reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) |
+        reinterpret_cast<uintptr_t>(norm_weight) | reinterpret_cast<uintptr_t>(residual)) & 15u) ||
       x_row_stride % 8)
     return MKV_ERR_MISALIGNED;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   LinearArgs a{reinterpret_cast<uint16_t*>(out), reinterpret_cast<const uint16_t*>(x),
-               reinterpret_cast<const uint16_t*>(w), x_row_stride, (int)rows, n, k, 1};
+               reinterpret_cast<const uint16_t*>(w), x_row_stride, (int)rows, n, k, 1,
+               reinterpret_cast<const uint16_t*>(norm_weight), eps, reinterpret_cast<const uint16_t*>(residual)};
   const int m_tiles = (int)(rows + 15) / 16;
   if (p.kind == 2) {
     switch (p.mt) {
@@ -363,12 +436,11 @@ extern "C" int mkv_linear(void* out, const void* x, int64_t x_row_stride, const 
   } else {
     a.m_groups = (m_tiles + p.mt - 1) / p.mt;
     if (act) {
-      if (p.mt == 2) launch_split<2, true>(a, p, s);
-      else launch_split<1, true>(a, p, s);
+      if (norm_weight) launch_rows<true, true>(a, p, s);
+      else launch_rows<true, false>(a, p, s);
     } else {
-      if (p.mt == 4) launch_split<4, false>(a, p, s);
-      else if (p.mt == 2) launch_split<2, false>(a, p, s);
-      else launch_split<1, false>(a, p, s);
+      if (norm_weight) launch_rows<false, true>(a, p, s);
+      else launch_rows<false, false>(a, p, s);
     }
   }
   return (int)hipGetLastError();

@@ -261,21 +261,33 @@ def silu_and_mul(x: torch.Tensor) -> torch.Tensor:
     return out
 
 
-def _own_product(x: torch.Tensor, w: torch.Tensor, n: int, act: int) -> bool:
-    """Whether mkv_linear takes x w^T: a few bf16 rows on the GPU with no
-    gradient to record, in sizes it shares out evenly."""
-    return (x.is_cuda and x.dtype == w.dtype == torch.bfloat16 and x.dim() == w.dim() == 2
-            and x.device == w.device and x.shape[1] == w.shape[1] and 0 < x.shape[0] <= 64
+def _own_weight(w: torch.Tensor, rows: int, n: int, act: int, norm: int = 0) -> bool:
+    """Whether mkv_linear takes the product of this many rows with w: bf16 on
+    the GPU, no gradient to record, in sizes it shares out evenly."""
+    return (w.is_cuda and w.dtype == torch.bfloat16 and w.dim() == 2 and w.is_contiguous()
+            and w.data_ptr() % 16 == 0 and not (torch.is_grad_enabled() and w.requires_grad)
+            and bool(_lib.query("mkv_linear_supported", rows, n, w.shape[1], act, norm, _lib.DTYPE_BF16)))
+
+
+def _own_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether mkv_linear reads x's rows as they are, for a w it takes."""
+    return (x.device == w.device and x.dtype == w.dtype and x.dim() == 2 and x.shape[1] == w.shape[1]
             and x.stride(1) == 1 and x.shape[1] <= x.stride(0) <= 1 << 20 and x.stride(0) % 8 == 0
-            and w.is_contiguous()
-            and (x.data_ptr() | w.data_ptr()) % 16 == 0
-            and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))
-            and bool(_lib.query("mkv_linear_supported", x.shape[0], n, x.shape[1], act, _dtype_code(x, "x"))))
+            and x.data_ptr() % 16 == 0 and not (torch.is_grad_enabled() and x.requires_grad))
 
 
-def _product(x: torch.Tensor, w: torch.Tensor, n: int, act: int) -> torch.Tensor:
-    out = torch.empty(x.shape[0], n, dtype=x.dtype, device=x.device)
-    _lib.call("mkv_linear", out.data_ptr(), x.data_ptr(), x.stride(0), w.data_ptr(), x.shape[0], n,
+def _own_product(x: torch.Tensor, w: torch.Tensor, n: int, act: int) -> bool:
+    return x.dim() == 2 and 0 < x.shape[0] <= 64 and _own_weight(w, x.shape[0], n, act) and _own_rows(x, w)
+
+
+def _product(x: torch.Tensor, w: torch.Tensor, n: int, act: int = 0, norm: torch.Tensor | None = None,
+             eps: float = 0.0, residual: torch.Tensor | None = None) -> torch.Tensor:
+    out = residual
+    if out is None:
+        out = torch.empty(x.shape[0], n, dtype=x.dtype, device=x.device)
+    _lib.call("mkv_linear", out.data_ptr(), x.data_ptr(), x.stride(0), w.data_ptr(),
+              norm.data_ptr() if norm is not None else None, float(eps),
+              residual.data_ptr() if residual is not None else None, x.shape[0], n,
               x.shape[1], act, _dtype_code(x, "x"), _stream(x.device))
     return out
 
@@ -283,7 +295,7 @@ def _product(x: torch.Tensor, w: torch.Tensor, n: int, act: int) -> torch.Tensor
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x w^T: for the few rows of a decode step one pass over the weights
     (mkv_linear), else torch's product."""
-    return _product(x, w, w.shape[0], 0) if _own_product(x, w, w.shape[0], 0) else F.linear(x, w)
+    return _product(x, w, w.shape[0]) if _own_product(x, w, w.shape[0], 0) else F.linear(x, w)
 
 
 def gated_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
@@ -385,15 +397,21 @@ class Qwen3Model(torch.nn.Module):
         attention metadata is the current mkv Context."""
         cfg = self.cfg
         Hq, Hkv, D = cfg.num_heads, cfg.num_kv_heads, cfg.head_dim
-        x = F.embedding(input_ids, self.embed)
-        residual = None
+        # The residual stream is residual, plus x where that is not None.
+        # Layers whose products all run on mkv_linear have their norms and
+        # residual additions in them (five launches a layer instead of seven).
+        x, residual = None, F.embedding(input_ids, self.embed)
         for li, lay in enumerate(self.layers):
-            if residual is None:
-                residual = x
-                h = rms_norm(x, lay["in_norm"], cfg.eps)
+            fused = self._fused_products(lay, residual)
+            if fused:
+                if x is not None:
+                    residual.add_(x)
+                    x = None
+                qkv = _product(residual, lay["qkv"], lay["qkv"].shape[0], 0, lay["in_norm"], cfg.eps)
             else:
-                h = rms_norm(x, lay["in_norm"], cfg.eps, residual)
-            qkv = linear(h, lay["qkv"])
+                h = rms_norm(residual, lay["in_norm"], cfg.eps) if x is None else \
+                    rms_norm(x, lay["in_norm"], cfg.eps, residual)
+                qkv = linear(h, lay["qkv"])
             att = lay["attn"]
             ctx = C.current_context()
             if self.fuse_decode_step and not ctx.is_prefill:
@@ -412,10 +430,25 @@ class Qwen3Model(torch.nn.Module):
                     eps=cfg.eps, kv_cache_dtype=att.kv_cache_dtype, k_scale=att.k_scale,
                     v_scale=att.v_scale, return_k=full_prefill)
                 o = self.attention(li, q, k, v)
+            if fused:
+                _product(o, lay["o"], cfg.hidden_size, residual=residual)
+                h = _product(residual, lay["gate_up"], cfg.intermediate_size, 1, lay["post_norm"], cfg.eps)
+                _product(h, lay["down"], cfg.hidden_size, residual=residual)
+                continue
             x = linear(o, lay["o"])
             h = rms_norm(x, lay["post_norm"], cfg.eps, residual)
             x = linear(gated_linear(h, lay["gate_up"]), lay["down"])
+        if x is None:
+            return rms_norm(residual, self.final_norm, cfg.eps)
         return rms_norm(x, self.final_norm, cfg.eps, residual)
+
+    def _fused_products(self, lay: dict, x: torch.Tensor) -> bool:
+        """Whether every product of the layer runs on mkv_linear for x's rows
+        (with 32768 or more features it takes no norm or residual)."""
+        rows, H, I = x.shape[0], self.cfg.hidden_size, self.cfg.intermediate_size
+        return (0 < rows <= 64 and max(lay["qkv"].shape[0], H) < 32768 and _own_rows(x, lay["qkv"])
+                and _own_weight(lay["qkv"], rows, lay["qkv"].shape[0], 0, 1) and _own_weight(lay["o"], rows, H, 0)
+                and _own_weight(lay["gate_up"], rows, I, 1, 1) and _own_weight(lay["down"], rows, H, 0))
 
     def logits(self, hidden: torch.Tensor) -> torch.Tensor:
         return linear(hidden, self.embed)

@@ -85,7 +85,7 @@ def test_linear(dev, rows, n, k, strided):
     feature tiles that do not fill them.  Bound: half an ulp of the output
     and k fp32 roundings of the sum of |x| |w|."""
     announce(f"linear {rows} x {n} x {k} strided={strided}")
-    assert _lib.query("mkv_linear_supported", rows, n, k, 0, _lib.DTYPE_BF16) == (n < 32768 or rows > 16)
+    assert _lib.query("mkv_linear_supported", rows, n, k, 0, 0, _lib.DTYPE_BF16) == (n < 32768 or rows > 16)
     g = torch.Generator().manual_seed(rows * 7 + n)
     w = torch.randn(n, k, generator=g).bfloat16().to(dev)
     x = torch.randn(rows, k + 8, generator=g).bfloat16().to(dev)
@@ -102,7 +102,7 @@ def test_gated_linear(dev, rows, inter, k):
     up are rounded to bf16 (half an ulp each, silu's slope at most 1.1) and
     so is the result, plus the products' fp32 sums."""
     announce(f"gated linear {rows} x {inter} x {k}")
-    assert _lib.query("mkv_linear_supported", rows, inter, k, 1, _lib.DTYPE_BF16)
+    assert _lib.query("mkv_linear_supported", rows, inter, k, 1, 0, _lib.DTYPE_BF16)
     g = torch.Generator().manual_seed(rows + inter)
     w = (torch.randn(2 * inter, k, generator=g) * 2 / k ** 0.5).bfloat16().to(dev)
     x = torch.randn(rows, k, generator=g).bfloat16().to(dev)
@@ -117,6 +117,87 @@ def test_gated_linear(dev, rows, inter, k):
     assert bool(((got - want).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("rows", [1, 17, 60])
+@pytest.mark.parametrize("n,k,act", [(16, 512, 0), (4096, 1024, 0), (48, 1536, 0), (32, 2048, 0), (48, 768, 1), (1024, 1024, 1)])
+def test_linear_with_norm(dev, rows, n, k, act):
+    """The product of normalised rows against the same of the norm kernel's
+    rows: equal, but for the order of the sum of squares, which moves 1 / rms
+    by 1e-6 at most and a term by one ulp (2^-8) where its rounding was that
+    nearly a tie, one in 10^3 of them.  Bound: 8 such terms, and an ulp of gate
+    and up and of the result."""
+    announce(f"linear with norm {rows} x {n} x {k} act {act}")
+    assert _lib.query("mkv_linear_supported", rows, n, k, act, 1, _lib.DTYPE_BF16)
+    g = torch.Generator().manual_seed(rows + n + k)
+    w = (torch.randn((1 + act) * n, k, generator=g) * 2 / k ** 0.5).bfloat16().to(dev)
+    x = (torch.randn(rows, k, generator=g) * torch.exp2(torch.randn(rows, 1, generator=g) * 3)).bfloat16().to(dev)
+    nw = (1 + 0.5 * torch.randn(k, generator=g)).bfloat16().to(dev)
+    got = E._product(x, w, n, act, nw, 1e-5).double()
+    h = E.rms_norm(x, nw, 1e-5)
+    want = (E.gated_linear if act else E.linear)(h, w).double()
+    p = h.double() @ w.double().t()
+    term = (h.double().abs().amax(-1, keepdim=True) * w.double().abs().amax(-1)) * 2.0 ** -8
+    e = 8 * term + _ulp(p)
+    if act:
+        (gate, up), (eg, eu) = p.chunk(2, -1), e.chunk(2, -1)
+        e = 1.1 * eg * (up.abs() + eu) + torch.nn.functional.silu(gate).abs() * eu
+    assert bool(((got - want).abs() <= e + _ulp(want)).all())
+    # the rows of the norm are the same but for those ties: 16 features pick
+    # out one element each
+    if not act and n == 16:
+        pick = torch.zeros(n, k).bfloat16().to(dev)
+        pick[torch.arange(n), torch.arange(n) * (k // n)] = 1
+        a, b = E._product(x, pick, n, 0, nw, 1e-5), h[:, :: k // n]
+        assert float((a != b).float().mean()) <= 0.02 and bool(((a - b).abs() <= 2.0 ** -7 * b.abs()).all())
+
+
+@pytest.mark.parametrize("rows", [1, 17, 60])
+@pytest.mark.parametrize("n,k", [(16, 512), (1024, 2048), (1024, 3072), (4096, 1024)])
+def test_linear_with_residual(dev, rows, n, k):
+    """The residual added in place equals the product alone added by torch."""
+    announce(f"linear with residual {rows} x {n} x {k}")
+    g = torch.Generator().manual_seed(rows + n)
+    w = torch.randn(n, k, generator=g).bfloat16().to(dev)
+    x = torch.randn(rows, k, generator=g).bfloat16().to(dev)
+    res = (20 * torch.randn(rows, n, generator=g)).bfloat16().to(dev)
+    want = E.linear(x, w) + res
+    got = E._product(x, w, n, residual=res)
+    assert got is res and torch.equal(got, want)
+
+
+def test_model_layers_with_and_without_fused_products(dev, monkeypatch):
+    """A model whose layers partly run on mkv_linear (a transposed weight is
+    left to torch) gives the hidden states of one that runs on torch alone,
+    to the bf16 rounding of each step (2^-8 over the 2 x 3 norms and sums)."""
+    from mkv import context as C
+    cfg = E.ModelConfig(vocab_size=512, hidden_size=1024, num_layers=3, intermediate_size=3072, max_position=64)
+    model = E.Qwen3Model(cfg, dev, block_size=16)
+    model.attach_kv_cache(8, "auto")
+    model.layers[1]["down"] = model.layers[1]["down"].t().contiguous().t()
+    ids = torch.arange(5, device=dev)
+    slots = torch.arange(5, device=dev) * 16
+    bt = torch.arange(5, dtype=torch.int32, device=dev)[:, None].contiguous()
+    calls = []
+
+    def run():
+        C.set_context(False, slot_mapping=slots, context_lens=torch.ones(5, dtype=torch.int64, device=dev),
+                      block_tables=bt)
+        try:
+            return model(ids, torch.zeros(5, dtype=torch.int64, device=dev), slots).double()
+        finally:
+            C.reset_context()
+
+    real = _lib.call
+    monkeypatch.setattr(_lib, "call", lambda name, *a: (calls.append(name), real(name, *a))[1])
+    got = run()
+    assert calls.count("mkv_linear") == 4 + 3 + 4  # (layer 1: qkv, o and the gated product, each by itself)
+    monkeypatch.setattr(E, "_own_weight", lambda *a: False)
+    want = run()
+    assert calls.count("mkv_linear") == 11
+    err = float((got - want).norm() / want.norm())
+    print("relative difference", err)
+    assert err < 6 * 2.0 ** -8
+
+
 def test_linear_leaves_other_products_to_torch(dev):
     """Sizes, types and layouts that mkv_linear does not take give torch's
     product: many rows, fp16, a transposed weight, a gradient to record."""
@@ -125,7 +206,7 @@ def test_linear_leaves_other_products_to_torch(dev):
     x = torch.randn(65, 1024, generator=g).to(dev)
     wb, xb = w.bfloat16(), x.bfloat16()
     wt = w.t().contiguous().bfloat16().t()
-    assert not any(_lib.query("mkv_linear_supported", m, n, k, 0, _lib.DTYPE_BF16)
+    assert not any(_lib.query("mkv_linear_supported", m, n, k, 0, 0, _lib.DTYPE_BF16)
                    for m, n, k in ((65, 64, 1024), (64, 6144, 1024), (16, 2048, 6144), (8, 2560, 2560),
                                    (1, 24, 1024), (1, 16, 16), (0, 16, 1024)))
     for a, b in ((xb, wb), (x[:8].half(), w.half()), (x[:8], w), (xb[:8], wt), (xb[:8, :40], wb[:, :40].contiguous())):
