@@ -2632,25 +2632,42 @@ MKV_DEV void merge_partials(const DecodeArgs& a, int64_t base, int nc, Slot slot
   for (int o = 32; o > 0; o >>= 1) l += __shfl_xor(l, o);
 }
 
+// The (sequence, query head) of a merge wave: a grid of (groups of kDecWaves
+// heads, sequences).  Both are scalars and come without a division, so the
+// sequence's metadata is one scalar round trip, all of it requested together:
+// a merge is a launch and a chain of round trips (stream-K steps, with a 64-bit
+// division and two round trips before: batch 48 of 10-3000 tokens, 16-bit,
+// head_dim 64 22.9 -> 22.2 us; batch 32 of 256-4096, FP8 per token and head,
+// 31.6 -> 30.8; batch 2 of 1209-2182, FP8, 18.3 -> 17.4; with the sequences
+// along x batch 256 of 1-5035 took 61.7 us, not 60.2 -> 59.9).
+dim3 merge_grid(int batch, int num_heads) {
+  const int y = batch < 32768 ? batch : 32768;
+  return dim3((unsigned)((num_heads + kDecWaves - 1) / kDecWaves), (unsigned)y, (unsigned)((batch + y - 1) / y));
+}
+MKV_DEV bool merge_item(const DecodeArgs& a, int& b, int& hq) {
+  b = (int)(blockIdx.z * gridDim.y + blockIdx.y);
+  hq = (int)blockIdx.x * kDecWaves + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  return b < a.batch && hq < a.num_heads;
+}
+
 __global__ __launch_bounds__(kDecWaves* kWave) void paged_decode_stream_merge_kernel(DecodeArgs a,
                                                                                      int kv_fp8) {
   const int lane = threadIdx.x & 63;
-  const int64_t wv = (int64_t)blockIdx.x * kDecWaves + (threadIdx.x >> 6);
-  if (wv >= (int64_t)a.batch * a.num_heads) return;
-  const int b = (int)(wv / a.num_heads);
-  const int hq = (int)(wv - (int64_t)b * a.num_heads);
-  const int kvh = hq / a.group, h = hq - kvh * a.group;
+  int b, hq;
+  if (!merge_item(a, b, hq)) return;
   const int p0 = a.sk_meta[b], n = a.sk_meta[b + 1] - p0;
   const int* meta = a.sk_meta + a.batch + 1 + 3 * b;
+  const int glo = meta[0], ghi = meta[1], s0 = meta[2];  // (0 for an empty sequence)
+  const float v_scale = kv_fp8 ? load_uniform_f32(a.v_scale) : 1.0f;
+  const int kvh = hq / a.group, h = hq - kvh * a.group;
   bool own;
   const int64_t off = (int64_t)b * a.out_stride + merge_out_offset(a, hq, h, lane, own);
   float o0 = 0.0f, o1 = 0.0f, l = 0.0f;
   if (n > 0) {
-    const int glo = meta[0], ghi = meta[1], s0 = meta[2];
     if (glo == ghi) return;  // written whole by the main kernel
     merge_partials(a, 0, ghi - glo + 1, [&](int i) { return merge_slot(a, glo, s0, glo + i, kvh, h); }, o0, o1, l);
   }
-  const float inv = l > 0.0f ? (kv_fp8 ? load_uniform_f32(a.v_scale) : 1.0f) / l : 0.0f;
+  const float inv = l > 0.0f ? v_scale / l : 0.0f;
   if (own) store_out2(a, off, o0 * inv, o1 * inv);
 }
 
@@ -2679,18 +2696,17 @@ paged_decode_mfma32_kernel(DecodeArgs a) {
 __global__ __launch_bounds__(kDecWaves* kWave) void paged_decode_merge_kernel(DecodeArgs a,
                                                                               int kv_fp8) {
   const int lane = threadIdx.x & 63;
-  const int64_t w = (int64_t)blockIdx.x * kDecWaves + (threadIdx.x >> 6);
-  if (w >= (int64_t)a.batch * a.num_heads) return;
-  const int b = (int)(w / a.num_heads);
-  const int hq = (int)(w - (int64_t)b * a.num_heads);
+  int b, hq;
+  if (!merge_item(a, b, hq)) return;
   int64_t L = load_index(a.context_lens, b, a.ctx_i64);
+  const float v_scale = kv_fp8 ? load_uniform_f32(a.v_scale) : 1.0f;
   const int64_t cap = (int64_t)a.idx.max_blocks << a.idx.bs_log2;
   L = L < 0 ? 0 : (L > cap ? cap : L);
   const int ns = L > 0 ? (int)((L + a.split_tokens - 1) / a.split_tokens) : 1;
   if (ns <= 1) return;
   float o0, o1, l;
   merge_partials(a, ((int64_t)b * a.num_heads + hq) * a.max_splits, ns, [](int i) { return i; }, o0, o1, l);
-  const float inv = l > 0.0f ? (kv_fp8 ? load_uniform_f32(a.v_scale) : 1.0f) / l : 0.0f;
+  const float inv = l > 0.0f ? v_scale / l : 0.0f;
   bool own;
   const int64_t off = (int64_t)b * a.out_stride + merge_out_offset(a, hq, hq % a.group, lane, own);
   if (own) store_out2(a, off, o0 * inv, o1 * inv);
@@ -3058,9 +3074,7 @@ int launch_route(DecodeArgs& a, int route, int fmt, int split_tokens, int max_bl
               : launch_stream<MKV_DTYPE_F16, false, PAIR>(a, lds_bucket, lds_bound, lds, s);
         break;
     }
-    const int64_t mitems = (int64_t)batch * a.num_heads;
-    hipLaunchKernelGGL(paged_decode_stream_merge_kernel,
-                       dim3((unsigned)((mitems + kDecWaves - 1) / kDecWaves)), dim3(kDecWaves * kWave), 0,
+    hipLaunchKernelGGL(paged_decode_stream_merge_kernel, merge_grid(batch, a.num_heads), dim3(kDecWaves * kWave), 0,
                        s, a, (int)fp8);
     return (int)hipGetLastError();
   }
@@ -3106,9 +3120,7 @@ int launch_route(DecodeArgs& a, int route, int fmt, int split_tokens, int max_bl
       break;
   }
   if (a.max_splits > 1) {
-    const int64_t mitems = (int64_t)batch * a.num_heads;
-    hipLaunchKernelGGL(paged_decode_merge_kernel, dim3((unsigned)((mitems + kDecWaves - 1) / kDecWaves)),
-                       block, 0, s, a, (int)fp8);
+    hipLaunchKernelGGL(paged_decode_merge_kernel, merge_grid(batch, a.num_heads), block, 0, s, a, (int)fp8);
   }
   return (int)hipGetLastError();
 }

@@ -385,3 +385,20 @@ def test_decode_fp32_tiles_and_merge_edges(dev, group, route):
     got = _run(dev, q, k, v, bt, ctx, 1 / math.sqrt(128), Hkv * group, Hkv, split_tokens=route)
     want = _oracle(q, k, v, bt, ctx, 1 / math.sqrt(128), Hkv * group, Hkv)
     assert_close_out(got, want, got.dtype, 2e-5)
+
+
+@pytest.mark.parametrize("group", [1, 5])
+def test_decode_merge_of_more_sequences_than_a_grid_row(dev, group):
+    """Split-K merges of 32,805 sequences, past the 32,768 of one row of the
+    merge's grid: the same 15 sequences over and over give the same results,
+    bit for bit (a sequence's splits and their order do not depend on the
+    batch)."""
+    announce(f"decode merge, 32805 sequences, group {group}")
+    ctx = torch.tensor([0, 1, 31, 32, 33, 40, 47, 48, 63, 64, 65, 80, 95, 96, 97], dtype=torch.int64)
+    Hkv, n = 1, 2187
+    q, k, v, bt, ctx, ks, vs = _case(77 + group, len(ctx), Hkv * group, Hkv, 16, 64, 7, torch.float32, ctx=ctx)
+    args = (1 / math.sqrt(128), Hkv * group, Hkv)
+    want = _run(dev, q, k, v, bt, ctx, *args, split_tokens=32)
+    assert_close_out(want, _oracle(q, k, v, bt, ctx, *args), want.dtype, 2e-5)
+    got = _run(dev, q.repeat(n, 1, 1), k, v, bt.repeat(n, 1), ctx.repeat(n), *args, split_tokens=32)
+    assert torch.equal(got, want.repeat(n, 1, 1))
