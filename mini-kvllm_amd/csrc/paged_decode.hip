@@ -2576,23 +2576,20 @@ MKV_DEV void merge_partials(const DecodeArgs& a, int64_t base, int nc, Slot slot
   o0 = o1 = l = 0.0f;
   auto row = [&](int sl) { return *reinterpret_cast<const f32x2*>(acc + (int64_t)sl * kHeadDim); };
   auto weight = [&](float wgt, int j) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wgt), j)); };
+  auto add = [&](bool in, float w, const f32x2& y) {
+    o0 = in ? o0 + w * y[0] : o0;
+    o1 = in ? o1 + w * y[1] : o1;
+  };
   // rows j0 .. of the partials held by the lanes (cnt of them), eight at a
-  // time; past the last one row 0 is read again and weighs nothing
+  // time; past the last one row 0 is read again and left out of the sums (by
+  // selection: a weight of 0 would make NaN of an infinity)
   auto rest = [&](int my_slot, float wgt, int j0, int cnt) {
     for (int j = j0; j < cnt; j += 8) {
       f32x2 y[8];
-      float w8[8];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const bool in = j + u < cnt;
-        y[u] = row(__builtin_amdgcn_readlane(my_slot, in ? j + u : 0));
-        w8[u] = in ? weight(wgt, j + u) : 0.0f;
-      }
+      for (int u = 0; u < 8; ++u) y[u] = row(__builtin_amdgcn_readlane(my_slot, j + u < cnt ? j + u : 0));
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        o0 += w8[u] * y[u][0];
-        o1 += w8[u] * y[u][1];
-      }
+      for (int u = 0; u < 8; ++u) add(j + u < cnt, weight(wgt, j + u < cnt ? j + u : 0), y[u]);
     }
   };
   if (nc <= kWave) {
@@ -2606,11 +2603,7 @@ MKV_DEV void merge_partials(const DecodeArgs& a, int64_t base, int nc, Slot slot
     const float wgt = lane < nc ? __builtin_amdgcn_exp2f(ml[0] - M) : 0.0f;
     l = wgt * ml[1];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {  // lanes past the last partial weigh nothing
-      const float w1 = weight(wgt, u);
-      o0 += w1 * x[u][0];
-      o1 += w1 * x[u][1];
-    }
+    for (int u = 0; u < 4; ++u) add(u < nc, weight(wgt, u), x[u]);
     rest(my_slot, wgt, 4, nc);
   } else {
     float M = kNegBig;

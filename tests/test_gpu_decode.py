@@ -402,3 +402,27 @@ def test_decode_merge_of_more_sequences_than_a_grid_row(dev, group):
     assert_close_out(want, _oracle(q, k, v, bt, ctx, *args), want.dtype, 2e-5)
     got = _run(dev, q.repeat(n, 1, 1), k, v, bt.repeat(n, 1), ctx.repeat(n), *args, split_tokens=32)
     assert torch.equal(got, want.repeat(n, 1, 1))
+
+
+@pytest.mark.parametrize("group", [2, 5])
+def test_decode_fp32_merge_keeps_infinities(dev, group):
+    """An infinity in the first or the last partial of a split-K merge, for
+    numbers of partials that do not fill the merge's groups of rows (1, 2, 3
+    of the first four; 5, 6, 13 with rows in groups of eight; 65, 70 past a
+    wave's 64 lanes): it comes out as that infinity and leaves every other dim
+    alone.  Bound as in test_decode_fp32_tiles_and_merge_edges."""
+    announce(f"decode fp32 merge with infinities, group {group}")
+    parts = [1, 2, 3, 5, 6, 13, 65, 70]
+    ctx = torch.tensor([32 * n for n in parts], dtype=torch.int64)
+    Hkv = 2
+    q, k, v, bt, ctx, _, _ = _case(950 + group, len(ctx), Hkv * group, Hkv, 32, 200, 70, torch.float32, ctx=ctx)
+    for b, n in enumerate(parts):
+        v[bt[b, 0], 3, 0, 5] = math.inf
+        v[bt[b, n - 1], 30, 1, 64] = -math.inf
+    args = (1 / math.sqrt(128), Hkv * group, Hkv)
+    got = _run(dev, q, k, v, bt, ctx, *args, split_tokens=32)
+    want = _oracle(q, k, v, bt, ctx, *args)
+    assert bool((want[:, :group, 5] == math.inf).all() and (want[:, group:, 64] == -math.inf).all())
+    inf = want.isinf()
+    assert int(inf.sum()) == len(parts) * Hkv * group and torch.equal(got[inf], want[inf].to(got.dtype))
+    assert_close_out(got[~inf], want[~inf], got.dtype, 2e-5)
