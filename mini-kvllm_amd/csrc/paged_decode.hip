@@ -2588,6 +2588,7 @@ MKV_DEV void merge_partials(const DecodeArgs& a, int64_t base, int nc, Slot slot
       f32x2 y[8];
 #pragma unroll
       for (int u = 0; u < 8; ++u) y[u] = row(__builtin_amdgcn_readlane(my_slot, j + u < cnt ? j + u : 0));
+      __builtin_amdgcn_sched_barrier(0);  // all eight in flight (the compiler split them in two fours)
 #pragma unroll
       for (int u = 0; u < 8; ++u) add(j + u < cnt, weight(wgt, j + u < cnt ? j + u : 0), y[u]);
     }
