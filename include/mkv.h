@@ -247,7 +247,10 @@ size_t mkv_paged_decode_workspace_size(int batch, int num_heads,
                                        int kv_dtype, int split_tokens);
 
 /* Tokens per split-K work item that mkv_paged_decode uses for these sizes
- * (split_tokens itself when it is > 0). */
+ * (split_tokens itself when it is > 0), with one query head per KV head.
+ * With more, and a table so wide that the partials would take more than
+ * MKV_NOALLOC_SCRATCH_BYTES, the default grows until they fit, up to 512
+ * tokens; mkv_paged_decode_workspace_size, which knows the heads, is exact. */
 int mkv_paged_decode_split_tokens(int batch, int num_kv_heads, int max_blocks,
                                   int block_size, int split_tokens);
 

@@ -2713,12 +2713,16 @@ int ilog2_exact(int v) {
   return l;
 }
 
-int default_split_tokens(int batch, int num_kv_heads, int max_blocks, int block_size) {
+// Bytes of split-K's partials for one split of every context: each query
+// head's accumulators and (m, l).
+size_t split_bytes(int64_t heads) { return (size_t)heads * (kHeadDim + 2) * sizeof(float); }
+
+int default_split_tokens(int batch, int num_kv_heads, int group, int max_blocks, int block_size) {
   // About 1024 work items (one wave per SIMD) from the longest context the
   // table allows, in splits of 64 tokens or more: a wave's start-up and its
   // partial cost as much as ~100 tokens.  At most 192 tokens, so that a batch
   // of uneven lengths stays balanced, except where whole sequences already
-  // fill the chip (there 512, which bounds the workspace).  Measured on fp32
+  // fill the chip (there 512).  Measured on fp32
   // caches, splits of 64 / 96 / 128 / 192 / 256 / 512 tokens: batch 1 of 700
   // tokens 14.1 / 16.3 / 18.4 / 21.9 / 25.8 / 43.0 us; batch 8 of 1000-3000
   // 38.2 / 34.5 / 39.2 / 29.9 / 31.7 / 47.7; batch 32 of 64-2048 48.8 / 46.1
@@ -2732,11 +2736,27 @@ int default_split_tokens(int batch, int num_kv_heads, int max_blocks, int block_
   const int64_t most = items < 1024 ? 192 : 512;
   if (st < 64) st = 64;
   if (st > most) st = most;
+  // The partials follow the table's width, whatever the contexts in it: past
+  // MKV_NOALLOC_SCRATCH_BYTES of them the splits grow until they fit, up to
+  // 512 tokens.  (Calls without a workspace keep this route that way: 32
+  // query heads, batch 64 of an 8192-token table, 44 MiB at 192 tokens, take
+  // 288.)  Splits of 192 / 256 / 320 / 512 tokens cost the same in wide
+  // tables that are full (batch 100 of 64-8192, 16 heads: 240 / 238 / 240 /
+  // 243 us; 64 of 64-4096, 32 heads: 129 / 128 / 127 / 135); where the
+  // contexts are short the shorter ones gain (batch 64 of 64-1000 in an
+  // 8192-token table: 43.5 / 49.7 / 57.2 / 48.1), so none grows sooner.
+  // (16-bit and quantised caches take this default past 8192 sequences or
+  // four KV heads a CU only, where it is 512 tokens or the whole context.)
+  const int64_t fit = items > 0 ? (int64_t)(MKV_NOALLOC_SCRATCH_BYTES / split_bytes(items * group)) : 0;
+  if ((max_len + st - 1) / st > (fit > 1 ? fit : 1)) {
+    const int64_t grown = fit > 0 ? ((max_len + fit - 1) / fit + 31) / 32 * 32 : 512;
+    st = grown < 512 ? grown : 512;
+  }
   return (int)st;
 }
 
-int resolve_split(int split_tokens, int batch, int num_kv_heads, int max_blocks, int block_size) {
-  if (split_tokens <= 0) return default_split_tokens(batch, num_kv_heads, max_blocks, block_size);
+int resolve_split(int split_tokens, int batch, int num_kv_heads, int group, int max_blocks, int block_size) {
+  if (split_tokens <= 0) return default_split_tokens(batch, num_kv_heads, group, max_blocks, block_size);
   return split_tokens;
 }
 
@@ -2803,7 +2823,7 @@ bool f32_small_group(int group, bool pair) { return group <= (pair ? 8 : 4); }
 size_t split_ws_bytes(int batch, int num_heads, int max_blocks, int block_size, int st) {
   const int64_t max_splits = ((int64_t)max_blocks * block_size + st - 1) / st;
   if (max_splits <= 1) return 0;
-  return (size_t)batch * num_heads * max_splits * (kHeadDim + 2) * sizeof(float);
+  return max_splits * split_bytes((int64_t)batch * num_heads);
 }
 
 // Kernel shape of a call: its KV heads and group as the kernels see them
@@ -2920,7 +2940,7 @@ size_t route_ws_bytes(int route, int batch, int num_heads, const KernelShape& ks
                       int block_size, int split_tokens) {
   if (route == kRouteWorkgroup) return 0;
   if (route == kRouteStream) return stream_ws_bytes(batch, ks.group);
-  const int st = resolve_split(split_tokens, batch, ks.kv_heads, max_blocks, block_size);
+  const int st = resolve_split(split_tokens, batch, ks.kv_heads, ks.group, max_blocks, block_size);
   return split_ws_bytes(batch, num_heads, max_blocks, block_size, st);
 }
 
@@ -2931,7 +2951,7 @@ using namespace mkv;
 
 extern "C" int mkv_paged_decode_split_tokens(int batch, int num_kv_heads, int max_blocks,
                                              int block_size, int split_tokens) {
-  return resolve_split(split_tokens, batch, num_kv_heads, max_blocks, block_size);
+  return resolve_split(split_tokens, batch, num_kv_heads, 1, max_blocks, block_size);
 }
 
 extern "C" int mkv_paged_decode_route(int batch, int num_heads, int num_kv_heads, int max_blocks,
@@ -3073,7 +3093,7 @@ int launch_route(DecodeArgs& a, int route, int fmt, int split_tokens, int max_bl
     return (int)hipGetLastError();
   }
 
-  const int st = resolve_split(split_tokens, batch, a.num_kv_heads, max_blocks, block_size);
+  const int st = resolve_split(split_tokens, batch, a.num_kv_heads, group, max_blocks, block_size);
   a.split_tokens = st;
   const int64_t max_len = (int64_t)max_blocks * block_size;
   a.max_splits = max_len > 0 ? (int)((max_len + st - 1) / st) : 1;

@@ -220,6 +220,36 @@ def test_fp32_decode_route_and_split():
     assert lib.mkv_paged_decode_split_tokens(128, 8, 32, 256, 0) == 512
 
 
+def test_fp32_split_workspace_in_wide_tables():
+    """split-K's default for fp32 caches, by the partials it makes: a call
+    whose partials fit the static scratch of mkv_paged_decode_noalloc with
+    4096 work items in splits of 64-512 tokens fits it still, none takes more
+    than the larger of that scratch and 512-token splits, and there is no
+    jump where whole sequences fill the chip (1024 items)."""
+    lib = _lib.load()
+    scratch = _lib.NOALLOC_SCRATCH_BYTES
+
+    def size(B, Hq, mb, split=_lib.DECODE_STREAM, bs=256, Hkv=8, D=128):
+        return lib.mkv_paged_decode_workspace_size(B, Hq, Hkv, mb, bs, D, _lib.DTYPE_F32, split)
+
+    for D in (128, 64):
+        for Hq in (8, 16, 32, 64, 128):
+            if Hq // 8 > (16 if D == 128 else 8):
+                continue
+            for B in (1, 3, 8, 20, 32, 50, 64, 100, 127, 128, 129, 200, 255, 256, 257, 600):
+                for mb in (1, 2, 3, 4, 8, 12, 16, 32, 33, 64, 128, 512):
+                    n, items = size(B, Hq, mb, D=D), B * 8 // (128 // D)
+                    want = -(-4096 // items)
+                    fine = min(512, max(64, -(-(-(-mb * 256 // want)) // 32) * 32))
+                    at_fine, at_512 = size(B, Hq, mb, fine, D=D), size(B, Hq, mb, 512, D=D)
+                    assert at_fine > scratch or n <= scratch, (D, Hq, B, mb, n, at_fine)
+                    assert n <= max(scratch, at_512), (D, Hq, B, mb, n, at_512)
+    # 32 query heads, 32768-token tables: 512-token splits on both sides of 1024 items
+    assert size(127, 32, 128) * 128 == size(128, 32, 128) * 127 == 127 * 128 * 32 * 64 * 520
+    # batch 64 of 8192 tokens: 29 splits of 288 tokens
+    assert size(64, 32, 32) == 64 * 32 * 29 * 520 <= scratch
+
+
 def test_decode_route_choice():
     """The library's schedule for split_tokens 0 (mkv_paged_decode_route on
     a 256-CU device), for the decode workloads that are measured, and the

@@ -160,3 +160,29 @@ def test_noalloc_default_route_falls_back_when_stream_slots_do_not_fit(dev, fmt)
                                  ksf, vsf)
         assert_close_out(got.cpu(), ref, got.dtype, tol)
         assert torch.count_nonzero(got[0].float()) == 0
+
+
+def test_noalloc_fp32_wide_table_keeps_split_k(dev):
+    """64 sequences of 32 query heads in 8192-token tables, fp32: split-K's
+    default keeps the partials within the scratch, so the call without a
+    workspace takes that route too and gives the same bytes."""
+    B, Hq, Hkv, bs, mb, N = 64, 32, 8, 256, 32, 40
+    announce("noalloc decode: fp32, 64 x 32 heads, 8192-token tables")
+    g = torch.Generator().manual_seed(77)
+    kc, vc, ks, vs, mode = _pools(dev, "f32", N, bs, Hkv, g)
+    bt = torch.randint(0, N, (B, mb), generator=g, dtype=torch.int32).to(dev)
+    ctx = torch.randint(0, mb * bs + 1, (B,), generator=g)
+    ctx[:4] = torch.tensor([0, 1, 288, 289])
+    ctx = ctx.to(dev)
+    q = torch.randn(B, Hq, D, generator=g).to(dev)
+    assert _lib.query("mkv_paged_decode_route", B, Hq, Hkv, mb, bs, D, _lib.DTYPE_F32, 0, 0) == _lib.ROUTE_SPLIT
+    need = _lib.query("mkv_paged_decode_workspace_size", B, Hq, Hkv, mb, bs, D, _lib.DTYPE_F32, 0)
+    assert need <= _lib.NOALLOC_SCRATCH_BYTES
+    ws = torch.empty(need, dtype=torch.uint8, device=dev)
+    want, got = torch.full_like(q, float("nan")), torch.full_like(q, float("nan"))
+    _call("mkv_paged_decode", want, q, kc, vc, ks, vs, mode, bt, ctx, Hq, Hkv, bs, 0, ws)
+    _call("mkv_paged_decode_noalloc", got, q, kc, vc, ks, vs, mode, bt, ctx, Hq, Hkv, bs, 0)
+    assert torch.equal(got, want) and bool(torch.isfinite(got).all())
+    ref = R.paged_decode_ref(q[:8].cpu().double(), kc.cpu(), vc.cpu(), bt[:8].cpu(), ctx[:8].cpu(),
+                             1.0 / math.sqrt(D), Hq, Hkv)
+    assert_close_out(got[:8].cpu(), ref, got.dtype, 2e-5)
