@@ -264,8 +264,8 @@ def silu_and_mul(x: torch.Tensor) -> torch.Tensor:
 def _own_weight(w: torch.Tensor, rows: int, n: int, act: int, norm: int = 0) -> bool:
     """Whether mkv_linear takes the product of this many rows with w: bf16 on
     the GPU, no gradient to record, in sizes it shares out evenly."""
-    return (w.is_cuda and w.dtype == torch.bfloat16 and w.dim() == 2 and w.is_contiguous()
-            and w.data_ptr() % 16 == 0 and not (torch.is_grad_enabled() and w.requires_grad)
+    return (w.is_cuda and w.dtype == torch.bfloat16 and w.dim() == 2 and w.shape[0] == (1 + act) * n
+            and w.is_contiguous() and w.data_ptr() % 16 == 0 and not (torch.is_grad_enabled() and w.requires_grad)
             and bool(_lib.query("mkv_linear_supported", rows, n, w.shape[1], act, norm, _lib.DTYPE_BF16)))
 
 
@@ -276,8 +276,8 @@ def _own_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
             and x.data_ptr() % 16 == 0 and not (torch.is_grad_enabled() and x.requires_grad))
 
 
-def _own_product(x: torch.Tensor, w: torch.Tensor, n: int, act: int) -> bool:
-    return x.dim() == 2 and 0 < x.shape[0] <= 64 and _own_weight(w, x.shape[0], n, act) and _own_rows(x, w)
+def _own_product(x: torch.Tensor, w: torch.Tensor, n: int, act: int, norm: int = 0) -> bool:
+    return x.dim() == 2 and 0 < x.shape[0] <= 64 and _own_weight(w, x.shape[0], n, act, norm) and _own_rows(x, w)
 
 
 def _product(x: torch.Tensor, w: torch.Tensor, n: int, act: int = 0, norm: torch.Tensor | None = None,
@@ -303,6 +303,33 @@ def gated_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     with the activation in its epilogue."""
     inter = w.shape[0] // 2
     return _product(x, w, inter, 1) if _own_product(x, w, inter, 1) else silu_and_mul(F.linear(x, w))
+
+
+def normed_linear(x: torch.Tensor | None, residual: torch.Tensor, norm: torch.Tensor, eps: float,
+                  w: torch.Tensor, act: int = 0) -> torch.Tensor:
+    """The (gated, with act) product of the RMS-normalised residual stream:
+    residual, plus x where that is not None (the sum is then left in
+    residual).  With nothing to add the norm runs inside the product where
+    mkv_linear takes it, else the add and the norm are a kernel ahead of it."""
+    n = w.shape[0] // (1 + act)
+    if (x is None and norm.device == w.device and norm.dtype == w.dtype and norm.shape == w.shape[1:]
+            and norm.is_contiguous() and norm.data_ptr() % 16 == 0 and _own_product(residual, w, n, act, 1)):
+        return _product(residual, w, n, act, norm, eps)
+    h = rms_norm(residual, norm, eps) if x is None else rms_norm(x, norm, eps, residual)
+    return gated_linear(h, w) if act else linear(h, w)
+
+
+def add_linear(residual: torch.Tensor, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor | None:
+    """residual += x w^T in the product's epilogue (None) where mkv_linear
+    takes the rows and the weight as they are, else the product, which is then
+    still to be added."""
+    if (residual.shape == (*x.shape[:-1], w.shape[0]) and residual.is_contiguous() and residual.dtype == w.dtype
+            and residual.device == w.device and residual.data_ptr() % 16 == 0
+            and w.shape[0] < 32768  # (more features take no residual)
+            and _own_product(x, w, w.shape[0], 0)):
+        _product(x, w, w.shape[0], residual=residual)
+        return None
+    return linear(x, w)
 
 
 class Qwen3Model(torch.nn.Module):
@@ -397,21 +424,12 @@ class Qwen3Model(torch.nn.Module):
         attention metadata is the current mkv Context."""
         cfg = self.cfg
         Hq, Hkv, D = cfg.num_heads, cfg.num_kv_heads, cfg.head_dim
-        # The residual stream is residual, plus x where that is not None.
-        # Layers whose products all run on mkv_linear have their norms and
-        # residual additions in them (five launches a layer instead of seven).
+        # The residual stream is residual, plus x where that is not None: in
+        # products that mkv_linear takes the norms and residual additions are
+        # part of them (five launches a layer instead of seven).
         x, residual = None, F.embedding(input_ids, self.embed)
         for li, lay in enumerate(self.layers):
-            fused = self._fused_products(lay, residual)
-            if fused:
-                if x is not None:
-                    residual.add_(x)
-                    x = None
-                qkv = _product(residual, lay["qkv"], lay["qkv"].shape[0], 0, lay["in_norm"], cfg.eps)
-            else:
-                h = rms_norm(residual, lay["in_norm"], cfg.eps) if x is None else \
-                    rms_norm(x, lay["in_norm"], cfg.eps, residual)
-                qkv = linear(h, lay["qkv"])
+            qkv = normed_linear(x, residual, lay["in_norm"], cfg.eps, lay["qkv"])
             att = lay["attn"]
             ctx = C.current_context()
             if self.fuse_decode_step and not ctx.is_prefill:
@@ -430,25 +448,12 @@ class Qwen3Model(torch.nn.Module):
                     eps=cfg.eps, kv_cache_dtype=att.kv_cache_dtype, k_scale=att.k_scale,
                     v_scale=att.v_scale, return_k=full_prefill)
                 o = self.attention(li, q, k, v)
-            if fused:
-                _product(o, lay["o"], cfg.hidden_size, residual=residual)
-                h = _product(residual, lay["gate_up"], cfg.intermediate_size, 1, lay["post_norm"], cfg.eps)
-                _product(h, lay["down"], cfg.hidden_size, residual=residual)
-                continue
-            x = linear(o, lay["o"])
-            h = rms_norm(x, lay["post_norm"], cfg.eps, residual)
-            x = linear(gated_linear(h, lay["gate_up"]), lay["down"])
+            x = add_linear(residual, o, lay["o"])
+            h = normed_linear(x, residual, lay["post_norm"], cfg.eps, lay["gate_up"], 1)
+            x = add_linear(residual, h, lay["down"])
         if x is None:
             return rms_norm(residual, self.final_norm, cfg.eps)
         return rms_norm(x, self.final_norm, cfg.eps, residual)
-
-    def _fused_products(self, lay: dict, x: torch.Tensor) -> bool:
-        """Whether every product of the layer runs on mkv_linear for x's rows
-        (with 32768 or more features it takes no norm or residual)."""
-        rows, H, I = x.shape[0], self.cfg.hidden_size, self.cfg.intermediate_size
-        return (0 < rows <= 64 and max(lay["qkv"].shape[0], H) < 32768 and _own_rows(x, lay["qkv"])
-                and _own_weight(lay["qkv"], rows, lay["qkv"].shape[0], 0, 1) and _own_weight(lay["o"], rows, H, 0)
-                and _own_weight(lay["gate_up"], rows, I, 1, 1) and _own_weight(lay["down"], rows, H, 0))
 
     def logits(self, hidden: torch.Tensor) -> torch.Tensor:
         return linear(hidden, self.embed)

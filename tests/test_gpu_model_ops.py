@@ -198,6 +198,61 @@ def test_model_layers_with_and_without_fused_products(dev, monkeypatch):
     assert err < 6 * 2.0 ** -8
 
 
+def test_model_takes_any_attention_rows(dev):
+    """The output of an overridden attention() may lie anyhow (every other
+    element of a wider buffer, transposed, off 16-byte alignment): the hidden
+    states are those of contiguous rows, to the bf16 rounding of each step (as
+    below).  Rows of another width than the output weight's, and a norm weight
+    at an odd address, give the errors that torch's product and the norm
+    kernel give, ahead of any product over them."""
+    from mkv import context as C
+    announce("model with attention rows in other layouts")
+    cfg = E.ModelConfig(vocab_size=512, hidden_size=1024, num_layers=2, intermediate_size=3072, max_position=64)
+
+    class Model(E.Qwen3Model):
+        fuse_decode_step = False
+        lay_out = staticmethod(lambda o: o)
+
+        def attention(self, li, q, k, v):
+            return self.lay_out(super().attention(li, q, k, v))
+
+    model = Model(cfg, dev, block_size=16)
+    model.attach_kv_cache(8, "auto")
+    ids, slots = torch.arange(5, device=dev), torch.arange(5, device=dev) * 16
+    bt = torch.arange(5, dtype=torch.int32, device=dev)[:, None].contiguous()
+
+    def run(lay_out):
+        model.lay_out = lay_out
+        C.set_context(False, slot_mapping=slots, context_lens=torch.ones(5, dtype=torch.int64, device=dev),
+                      block_tables=bt)
+        try:
+            return model(ids, torch.zeros(5, dtype=torch.int64, device=dev), slots).double()
+        finally:
+            C.reset_context()
+
+    def spread(o):
+        wide = torch.full((o.shape[0], 2 * o.shape[1]), 7.0, dtype=o.dtype, device=dev)
+        wide[:, ::2] = o
+        return wide[:, ::2]
+
+    def off(o):
+        buf = torch.zeros(o.shape[0], o.shape[1] + 8, dtype=o.dtype, device=dev)
+        buf[:, 1:o.shape[1] + 1] = o
+        return buf[:, 1:o.shape[1] + 1]
+
+    want = run(lambda o: o)
+    for lay_out in (spread, lambda o: o.t().contiguous().t(), off):
+        got = run(lay_out)
+        assert float((got - want).norm() / want.norm()) < 4 * 2.0 ** -8
+    for width in (1024, 4096):
+        with pytest.raises(RuntimeError):
+            run(lambda o: torch.zeros(5, width, dtype=o.dtype, device=dev))
+    buf = torch.ones(1032, dtype=torch.bfloat16, device=dev)
+    model.layers[0]["post_norm"] = buf[1:1025]
+    with pytest.raises(_lib.MkvError, match="mkv_rmsnorm"):
+        run(lambda o: o)
+
+
 def test_linear_leaves_other_products_to_torch(dev):
     """Sizes, types and layouts that mkv_linear does not take give torch's
     product: many rows, fp16, a transposed weight, a gradient to record."""
