@@ -35,6 +35,7 @@ from dataclasses import dataclass, field
 
 import torch
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 
 from . import _lib
 from . import context as C
@@ -269,15 +270,29 @@ def _own_weight(w: torch.Tensor, rows: int, n: int, act: int, norm: int = 0) -> 
             and bool(_lib.query("mkv_linear_supported", rows, n, w.shape[1], act, norm, _lib.DTYPE_BF16)))
 
 
+def _plain(*tensors: torch.Tensor) -> bool:
+    """Whether a kernel on the tensors' memory is all that a product of them
+    means: nothing traces or intercepts it (torch.compile, jit, dispatch
+    modes), and no tensor is a subclass's, one of a function transform's
+    (vmap, jvp) or carries a forward-mode tangent."""
+    return (not torch.compiler.is_compiling() and not torch.jit.is_tracing()
+            and torch._C._len_torch_dispatch_stack() == 0
+            and all(type(t) in (torch.Tensor, torch.nn.Parameter)
+                    and not torch._C._functorch.is_functorch_wrapped_tensor(t)
+                    and forward_ad.unpack_dual(t).tangent is None for t in tensors))
+
+
 def _own_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether mkv_linear reads x's rows as they are, for a w it takes."""
-    return (x.device == w.device and x.dtype == w.dtype and x.dim() == 2 and x.shape[1] == w.shape[1]
+    """Whether mkv_linear reads x's rows as they are, for a w it takes (on the
+    current device: it launches there)."""
+    return (x.device == w.device and x.get_device() == torch.cuda.current_device() and x.dtype == w.dtype and x.dim() == 2 and x.shape[1] == w.shape[1]
             and x.stride(1) == 1 and x.shape[1] <= x.stride(0) <= 1 << 20 and x.stride(0) % 8 == 0
             and x.data_ptr() % 16 == 0 and not (torch.is_grad_enabled() and x.requires_grad))
 
 
 def _own_product(x: torch.Tensor, w: torch.Tensor, n: int, act: int, norm: int = 0) -> bool:
-    return x.dim() == 2 and 0 < x.shape[0] <= 64 and _own_weight(w, x.shape[0], n, act, norm) and _own_rows(x, w)
+    return (_plain(x, w) and x.dim() == 2 and 0 < x.shape[0] <= 64
+            and _own_weight(w, x.shape[0], n, act, norm) and _own_rows(x, w))
 
 
 def _product(x: torch.Tensor, w: torch.Tensor, n: int, act: int = 0, norm: torch.Tensor | None = None,

@@ -9,6 +9,7 @@ from __future__ import annotations
 import random
 
 import pytest
+import torch
 
 from mkv import engine as E
 
@@ -131,3 +132,42 @@ def test_request_larger_than_the_pool_is_refused():
     sched.add(fits)
     _run(sched, [fits], bs)
     assert fits.num_generated == 4
+
+
+def test_products_under_transforms_are_left_to_torch():
+    """The engine's products run on tensors' memory only where that is all
+    they mean: not with a forward-mode tangent, inside vmap / jvp, on a
+    subclass, under a dispatch mode (fake tensors, make_fx) or a trace."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.autograd import forward_ad
+    from torch.fx.experimental.proxy_tensor import make_fx
+
+    class Sub(torch.Tensor):
+        pass
+
+    x, w = torch.randn(3, 8), torch.nn.Parameter(torch.randn(4, 8))
+    seen = []
+
+    def f(t):
+        seen.append(E._plain(t, w))
+        return E.linear(t, w)
+
+    want = torch.nn.functional.linear(x, w)
+    f(x)
+    with torch.no_grad():
+        f(x)
+    assert seen == [True, True] and E._plain(w)
+    seen.clear()
+    with forward_ad.dual_level():
+        y = forward_ad.unpack_dual(f(forward_ad.make_dual(x, 2 * x)))
+        assert torch.allclose(y.primal, want) and torch.allclose(y.tangent, 2 * want)
+    _, tangent = torch.func.jvp(f, (x,), (2 * x,))
+    assert torch.allclose(tangent, 2 * want)
+    assert torch.allclose(torch.func.vmap(f)(x[:, None])[:, 0], want)
+    with FakeTensorMode(allow_non_fake_inputs=True):
+        assert f(torch.empty(5, 8)).shape == (5, 4)
+    assert torch.allclose(f(x.as_subclass(Sub)), want)
+    assert torch.allclose(make_fx(f)(x)(2 * x), 2 * want)
+    w = w.detach()
+    assert torch.allclose(torch.jit.trace(f, x, check_trace=False)(2 * x), 2 * want)
+    assert len(seen) == 7 and not any(seen)

@@ -253,6 +253,33 @@ def test_model_takes_any_attention_rows(dev):
         run(lambda o: o)
 
 
+def test_logits_keep_transforms_and_the_current_device(dev, monkeypatch):
+    """The LM head under forward mode and vmap gives torch's tangent and
+    rows, and where another device is the current one torch's product."""
+    from torch.autograd import forward_ad
+    announce("logits under jvp, vmap and another current device")
+    cfg = E.ModelConfig(vocab_size=512, hidden_size=1024, num_layers=1, intermediate_size=512, max_position=64)
+    model = E.Qwen3Model(cfg, dev, block_size=16)
+    g = torch.Generator().manual_seed(5)
+    x, t = (torch.randn(20, 1024, generator=g).bfloat16().to(dev) for _ in range(2))
+    calls = []
+    real = _lib.call
+    monkeypatch.setattr(_lib, "call", lambda name, *a: (calls.append(name), real(name, *a))[1])
+    torch_rows = torch.nn.functional.linear(x, model.embed)
+    with forward_ad.dual_level():
+        y = forward_ad.unpack_dual(model.logits(forward_ad.make_dual(x, t)))
+        assert torch.equal(y.primal, torch_rows)
+        assert torch.equal(y.tangent, torch.nn.functional.linear(t, model.embed))
+    rows = torch.func.vmap(model.logits)(x.view(4, 5, 1024)).view(20, 512)
+    assert float((rows.double() - torch_rows.double()).norm() / torch_rows.double().norm()) < 2.0 ** -8
+    with monkeypatch.context() as m:
+        m.setattr(torch.cuda, "current_device", lambda: 1 + dev.index if dev.index is not None else 1)
+        assert torch.equal(model.logits(x), torch_rows)
+    assert calls == []
+    model.logits(x)
+    assert calls == ["mkv_linear"]
+
+
 def test_linear_leaves_other_products_to_torch(dev):
     """Sizes, types and layouts that mkv_linear does not take give torch's
     product: many rows, fp16, a transposed weight, a gradient to record."""
