@@ -540,7 +540,7 @@ int mkv_silu_mul(void* out, const void* x, int64_t x_row_stride, int64_t rows,
  * waves; not where the library is as fast); others return MKV_ERR_BAD_SHAPE,
  * as do rows of x more than 2^20 elements apart.  norm_weight (k,) non-NULL
  * (norm 1 in the query): the product of the rows that mkv_rmsnorm makes of x
- * without a residual.  residual (rows, n) non-NULL (act 0, fewer than 32768
+ * without a residual (k up to its 2048).  residual (rows, n) non-NULL (act 0, fewer than 32768
  * features; it may be out): out = round(round(product) + residual). */
 int mkv_linear_supported(int64_t rows, int n, int k, int act, int norm, int dtype);
 int mkv_linear(void* out, const void* x, int64_t x_row_stride, const void* w,

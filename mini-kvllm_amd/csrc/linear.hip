@@ -26,6 +26,7 @@ namespace mkv {
 namespace {
 
 constexpr int kLinMaxRows = 64;
+constexpr int kNormMaxK = 2048;  // mkv_rmsnorm's
 constexpr int64_t kLinMaxStride = (int64_t)1 << 20;  // x's offsets are 32 bits
 constexpr int kCus = 256;
 constexpr int kXcds = 8;
@@ -332,6 +333,7 @@ struct LinearPlan {
 LinearPlan plan_linear(int64_t rows, int n, int k, int act, int norm) {
   LinearPlan p{0, 0, 0, 0};
   if (rows < 1 || rows > kLinMaxRows || n < 16 || n % 16 || k < 32 || k % 32) return p;
+  if (norm && k > kNormMaxK) return p;
   const int m_tiles = (int)(rows + 15) / 16, n_tiles = n / 16;
   // Streaming from 8 feature tiles a CU on (its offsets are 32 bits), for more
   // than 16 rows: at most 16 are as fast or faster in the library (151936 x

@@ -250,6 +250,18 @@ def test_fp32_split_workspace_in_wide_tables():
     assert size(64, 32, 32) == 64 * 32 * 29 * 520 <= scratch
 
 
+def test_normalised_products_are_as_wide_as_the_norm_kernel():
+    """mkv_linear's norm stands for mkv_rmsnorm's, which takes rows of up to
+    2048: a wider model is refused at its first norm, not at its last, with
+    every layer's K and V already in the cache."""
+    lib = _lib.load()
+    for rows in (1, 16, 60):
+        assert lib.mkv_linear_supported(rows, 1024, 2048, 0, 1, _lib.DTYPE_BF16) == 1
+        assert lib.mkv_linear_supported(rows, 1024, 3072, 0, 0, _lib.DTYPE_BF16) == 1
+        for act in (0, 1):
+            assert lib.mkv_linear_supported(rows, 1024, 3072, act, 1, _lib.DTYPE_BF16) == 0
+
+
 def test_decode_route_choice():
     """The library's schedule for split_tokens 0 (mkv_paged_decode_route on
     a 256-CU device), for the decode workloads that are measured, and the
