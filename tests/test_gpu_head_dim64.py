@@ -243,6 +243,38 @@ def test_flash_prefill_head_dim64(dev, dtype, group):
     assert_close_out(got, want, got.dtype, 2e-3)
 
 
+@pytest.mark.parametrize("paged", [True, False])
+@pytest.mark.parametrize("group,copies", [(4, 2), (4, 9), (8, 5)])
+def test_prefill_head_dim64_fp32_workgroup_forms(dev, paged, group, copies):
+    """fp32 caches in the launch forms for three workgroups a CU and for 64
+    rows a workgroup (4096 or more of 32 rows: the batch is repeated over one
+    pool), on paired heads, with an absent block.  Bound: a sum of n <= 260
+    fp32 products of N(0, 1) values in any order is within n ulps of its
+    terms' sum; measured errors are 1e-6."""
+    announce(f"prefill head_dim 64 fp32 forms: paged {paged}, group {group} x {copies}")
+    Hkv = 8
+    Hq, n = Hkv * group, 11
+    qlen = [1, 2, 15, 16, 17, 31, 33, 64, 65, 97, 130]
+    prior = [0, 31, 1, 16, 15, 0, 95, 0, 31, 0, 130] if paged else [0] * n
+    q, dp, hp, bt, ctx, cu, pos = _prefill_case(660 + group, "f32", Hq, Hkv, 16, prior, qlen, dev,
+                                                holes=[(10, 5)] if paged else [])
+    sc, T = 1 / math.sqrt(D), q.shape[0]
+    off = torch.arange(copies, dtype=torch.int32).repeat_interleave(n) * T
+    cus = torch.cat([cu[:-1].repeat(copies) + off, torch.tensor([copies * T], dtype=torch.int32)])
+    qs = q.repeat(copies, 1, 1).to(dev)
+    if paged:
+        want = R.paged_prefill_ref(q.double(), hp[0], hp[1], bt, ctx, cu, pos, sc, Hq, Hkv, None, None)
+        got = A.paged_attention_prefill_triton(qs, dp[0], dp[1], bt.repeat(copies, 1).to(dev),
+                                               ctx.repeat(copies).to(dev), cus.to(dev), pos.repeat(copies).to(dev),
+                                               sc, Hq, Hkv, D, 16).cpu()
+    else:
+        k, v = hp[0].flatten(0, 1)[:T], hp[1].flatten(0, 1)[:T]
+        want = R.flash_prefill_ref(q.double(), k.double(), v.double(), cu, sc, Hq, Hkv)
+        got = mkv.flash_attention_prefill(qs, k.repeat(copies, 1, 1).to(dev), v.repeat(copies, 1, 1).to(dev),
+                                          cus.to(dev), sc, Hq, Hkv, D).cpu()
+    assert_close_out(got, want.repeat(copies, 1, 1), got.dtype, 2e-5)
+
+
 @pytest.mark.parametrize("mode", ["auto", "fp8_per_tensor", "fp8_per_token_head"])
 def test_attention_layer_head_dim64_full_then_chunked_then_decode(dev, mode):
     """The Llama-3.2-1B attention shape through Attention.forward: three

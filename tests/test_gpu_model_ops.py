@@ -100,7 +100,9 @@ def test_linear(dev, rows, n, k, strided):
 def test_gated_linear(dev, rows, inter, k):
     """The gated product against silu(gate) * up in 64 bits.  Bound: gate and
     up are rounded to bf16 (half an ulp each, silu's slope at most 1.1) and
-    so is the result, plus the products' fp32 sums."""
+    so is the result, plus the products' fp32 sums.  The result's ulp is that
+    of what is rounded: of 64-bit 3.9955, 4.016 may be, half of 4's ulp away
+    (torch's product and mkv_silu_mul give the same value there)."""
     announce(f"gated linear {rows} x {inter} x {k}")
     assert _lib.query("mkv_linear_supported", rows, inter, k, 1, 0, _lib.DTYPE_BF16)
     g = torch.Generator().manual_seed(rows + inter)
@@ -113,7 +115,8 @@ def test_gated_linear(dev, rows, inter, k):
     eg, eu = e.chunk(2, -1)
     silu = torch.nn.functional.silu(gate)
     want = silu * up
-    bound = 1.1 * eg * (up.abs() + eu) + silu.abs() * eu + 0.5 * _ulp(want) * 1.01 + 1e-6 * want.abs()
+    bound = 1.1 * eg * (up.abs() + eu) + silu.abs() * eu + 1e-6 * want.abs()
+    bound = bound + 0.5 * _ulp(want.abs() + bound) * 1.01
     assert bool(((got - want).abs() <= bound).all())
 
 
@@ -196,6 +199,30 @@ def test_model_layers_with_and_without_fused_products(dev, monkeypatch):
     err = float((got - want).norm() / want.norm())
     print("relative difference", err)
     assert err < 6 * 2.0 ** -8
+
+
+# Sizes in the forms that the tests above leave out: k in 4, 8 and 16 parts of
+# 4 or 6 steps, 32 and 64 rows a workgroup, at the fewest and the most features
+# that take each.
+_WIDE = [(64, 2048, 2048), (33, 2720, 2048), (17, 4096, 2048), (33, 2048, 512), (31, 16384, 512), (64, 2048, 768),
+         (17, 4112, 768), (48, 2048, 1536), (32, 5456, 1536), (64, 4096, 512), (33, 10752, 512), (48, 5456, 1024)]
+
+
+@pytest.mark.parametrize("rows,n,k", _WIDE)
+def test_linear_wide_forms(dev, rows, n, k):
+    test_linear(dev, rows, n, k, True)
+
+
+@pytest.mark.parametrize("rows,n,k", _WIDE + [(1, 16, 2048), (16, 32, 4096), (1, 16, 768), (16, 32, 1536)])
+def test_gated_linear_wide_forms(dev, rows, n, k):
+    test_gated_linear(dev, rows, n, k)
+
+
+@pytest.mark.parametrize("act,rows,n,k", [(0, *s) for s in _WIDE + [(1, 16, 768)]] +
+                         [(1, *s) for s in _WIDE + [(1, 16, 2048), (1, 16, 512), (1, 16, 1536),
+                                                    (33, 3072, 1024), (60, 3072, 1024), (64, 3072, 1024)]])
+def test_linear_with_norm_wide_forms(dev, act, rows, n, k):
+    test_linear_with_norm(dev, rows, n, k, act)
 
 
 def test_model_takes_any_attention_rows(dev):

@@ -48,6 +48,17 @@ def test_decode_and_prefill_kernels_do_not_spill(resources):
           f"in {len(sgpr)}")
 
 
+def test_linear_kernels_do_not_spill(resources):
+    """The decode step's products: every form of the split kernel (row tiles,
+    k-steps, gated, normalised) and of the streaming one."""
+    hot = {k: v for k, v in resources.items() if "linear_split" in k or "linear_stream" in k}
+    names = _demangle(list(hot))
+    assert len(hot) >= 20, f"expected every instantiation, found {len(hot)}"
+    bad = {names[k]: (v.get("VGPRs Spill"), v.get("ScratchSize")) for k, v in hot.items()
+           if v.get("VGPRs Spill", -1) or v.get("ScratchSize", -1)}
+    assert not bad, f"VGPR spills / scratch bytes per lane: {bad}"
+
+
 def test_headline_decode_kernel_residency(resources):
     """The batch-256 FP8 decode kernel (stream-K, groups of up to 4 query
     heads) holds two waves per SIMD: its persistent grid is sized for that."""
