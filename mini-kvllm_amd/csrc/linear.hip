@@ -30,6 +30,7 @@ constexpr int kNormMaxK = 2048;  // mkv_rmsnorm's
 constexpr int64_t kLinMaxStride = (int64_t)1 << 20;  // x's offsets are 32 bits
 constexpr int kCus = 256;
 constexpr int kXcds = 8;
+constexpr size_t kLdsPerCu = 160 * 1024;
 
 struct LinearArgs {
   uint16_t* out;      // (rows, n)
@@ -330,6 +331,14 @@ struct LinearPlan {
   int mt, waves, blk;
 };
 
+// LDS of a split workgroup: x's parts (normalised: and the waves' sums of
+// squares), then the waves' sums in their place.
+size_t split_lds(const LinearPlan& p, int act, int norm) {
+  const size_t sums = (size_t)p.waves * (act ? 2 : 1) * p.mt * 1024;
+  const size_t x = (size_t)p.waves * p.mt * (16 * p.blk * 64 + (norm ? 64 : 0));
+  return sums > x ? sums : x;
+}
+
 LinearPlan plan_linear(int64_t rows, int n, int k, int act, int norm) {
   LinearPlan p{0, 0, 0, 0};
   if (rows < 1 || rows > kLinMaxRows || n < 16 || n % 16 || k < 32 || k % 32) return p;
@@ -372,15 +381,22 @@ LinearPlan plan_linear(int64_t rows, int n, int k, int act, int norm) {
   if (act && p.mt == 4) p.mt = 2;
   if ((p.waves == 16 || p.blk == 6) && p.mt == 4) p.mt = 2;
   if (act && norm && p.blk == 6) p.mt = 1;  // (two row tiles do not fit the registers)
+  // Not where one workgroup fills a CU's LDS and there are more of them than
+  // CUs: the few of the second round take as long as all of the first.  Here and
+  // in the library, us: 2560 x 1536 at 48 rows 10.4 and 9.5, 1536 x 3072 at 48
+  // 13.3 / 10.2 and gated 19.9 / 13.7, normalised 2560 x 2048 at 33 19.8 / 15.6 and
+  // 4608 x 1024 at 33 17.2 / 15.1; but plain 4608 x 1024 at 33 10.4 / 11.8.
+  // Two a CU hide each other, in more rounds too: 3072 x 2048 at 32 rows 8.8 /
+  // 11.5, 24576 x 512 at 16 8.7 / 12.6, 8192 x 2048 normalised at 16 16.1 / 18.4.
+  const int64_t wgs = (int64_t)n_tiles * ((m_tiles + p.mt - 1) / p.mt);
+  if (wgs > kCus && 2 * split_lds(p, act, norm) > kLdsPerCu && (k > 1024 || norm)) return LinearPlan{0, 0, 0, 0};
   return p;
 }
 
 template <int MT, bool ACT, bool NORM>
 void launch_split(const LinearArgs& a, const LinearPlan& p, hipStream_t s) {
   const dim3 grid((unsigned)(a.n / 16 * a.m_groups)), block(p.waves * kWave);
-  const size_t sums = (size_t)p.waves * (ACT ? 2 : 1) * MT * 1024;
-  const size_t x = (size_t)p.waves * MT * (16 * p.blk * 64 + (NORM ? 64 : 0));
-  const size_t lds = sums > x ? sums : x;
+  const size_t lds = split_lds(p, ACT, NORM);
   constexpr bool kFour = MT == 4 || (MT == 2 && ACT && NORM);  // plan_linear's
   if (kFour || p.blk == 4)
     hipLaunchKernelGGL((linear_split_kernel<MT, 4, ACT, NORM>), grid, block, lds, s, a);

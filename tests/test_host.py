@@ -262,6 +262,23 @@ def test_normalised_products_are_as_wide_as_the_norm_kernel():
             assert lib.mkv_linear_supported(rows, 1024, 3072, act, 1, _lib.DTYPE_BF16) == 0
 
 
+def test_products_leave_a_second_round_to_the_library():
+    """mkv_linear takes no product whose workgroups each fill a CU's LDS and
+    outnumber the CUs (plain ones of k to 1024 apart), where the library is
+    faster; one workgroup a CU, and more with two of them a CU, it takes."""
+    lib = _lib.load()
+
+    def taken(rows, n, k, act=0, norm=0):
+        return lib.mkv_linear_supported(rows, n, k, act, norm, _lib.DTYPE_BF16)
+
+    for rows, n, k in ((33, 2560, 1536), (48, 1536, 3072), (17, 2560, 3072), (16, 4352, 3072)):
+        assert not taken(rows, n, k) and not taken(rows, n, k, 1)
+    assert not taken(33, 2560, 2048, 0, 1) and not taken(33, 4608, 1024, 0, 1) and not taken(33, 2560, 1536, 0, 1)
+    assert taken(33, 4608, 1024) and taken(32, 4096, 1536) and taken(64, 4096, 1024, 0, 1)
+    assert taken(16, 4096, 3072) and taken(64, 1024, 3072) and taken(64, 3072, 1024, 1, 1)
+    assert taken(32, 3072, 2048) and taken(16, 24576, 512) and taken(16, 8192, 2048, 0, 1)
+
+
 def test_decode_route_choice():
     """The library's schedule for split_tokens 0 (mkv_paged_decode_route on
     a 256-CU device), for the decode workloads that are measured, and the
