@@ -537,7 +537,8 @@ int mkv_silu_mul(void* out, const void* x, int64_t x_row_stride, int64_t rows,
  * round(silu(gate) * up) on gate and up rounded to bf16 (what mkv_silu_mul
  * gives on the product).  mkv_linear_supported says whether a product's sizes
  * are taken (bf16, n a multiple of 16, k shared out evenly over 4, 8 or 16
- * waves; not where the library is as fast); others return MKV_ERR_BAD_SHAPE,
+ * waves, from 32768 features on k 512, 1024, 1536 or 2048; not where the
+ * library is as fast); others return MKV_ERR_BAD_SHAPE,
  * as do rows of x more than 2^20 elements apart.  norm_weight (k,) non-NULL
  * (norm 1 in the query): the product of the rows that mkv_rmsnorm makes of x
  * without a residual (k up to its 2048).  residual (rows, n) non-NULL (act 0, fewer than 32768

@@ -230,21 +230,23 @@ __global__ __launch_bounds__(1024) void linear_split_kernel(LinearArgs a) {
 // ---------------------------------------------------------------------------
 // Streaming form, for products with many more feature tiles than CUs (an LM
 // head): one 8-wave workgroup a CU takes a contiguous range of feature tiles.
-// Each wave keeps its eighth of x (4 k-steps of every row) in registers and
-// streams its eighth of the tiles' weights through a ring of three pairs of
-// tiles, two pairs (128 KB a CU) in flight ahead of the one it multiplies; the
-// waves' sums of a pair meet in LDS (double-buffered, one barrier a pair that
-// leaves the loads in flight), where wave w joins tile w / 4, rows 16 (w % 4).
-// 311 MB of weights: 63 us for one row, 78 for 60 (the writes of 18 MB of
-// logits); plain loads, since non-temporal ones took 68 and 88.
+// Each wave keeps its eighth of x (STEPS k-steps of every row) in registers and
+// streams its eighth of the tiles' weights through a ring of three groups of
+// tiles (pairs, single ones past k 1024), two groups (128 KB a CU for k 1024 and
+// 2048) in flight ahead of the one it multiplies; the waves' sums of a group meet
+// in LDS (double-buffered, one barrier a group that leaves the loads in flight),
+// where wave w joins tile w / 4, rows 16 (w % 4).
+// 151936 x 1024 (311 MB of weights): 63 us for one row, 78 for 60 (the writes of
+// 18 MB of logits); plain loads, since non-temporal ones took 68 and 88.
 // ---------------------------------------------------------------------------
 constexpr int kStreamWaves = 8;
-constexpr int kStreamSteps = 4;                              // k-steps of a wave
-constexpr int kStreamK = 32 * kStreamSteps * kStreamWaves;  // 1024
 
-template <int MT>
+template <int MT, int STEPS>
 __global__ __launch_bounds__(kStreamWaves* kWave) __attribute__((amdgpu_waves_per_eu(2))) void linear_stream_kernel(
     LinearArgs a) {
+  static_assert(STEPS % 2 == 0, "step_off goes by pairs of k-steps");
+  constexpr int kK = 32 * STEPS * kStreamWaves;
+  constexpr int TP = STEPS <= 4 ? 2 : 1;  // tiles of a group
   extern __shared__ __align__(16) char smem[];
   f32x4* part = reinterpret_cast<f32x4*>(smem);  // [2][wave][tile][MT][lane]
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -253,75 +255,76 @@ __global__ __launch_bounds__(kStreamWaves* kWave) __attribute__((amdgpu_waves_pe
   const int nwg = gridDim.x;
   const int b = nwg % kXcds == 0 ? (blockIdx.x % kXcds) * (nwg / kXcds) + blockIdx.x / kXcds : blockIdx.x;
   const int t0 = (int)((int64_t)tiles * b / nwg), t1 = (int)((int64_t)tiles * (b + 1) / nwg);
-  const int pairs = (t1 - t0 + 1) / 2;
-  if (pairs == 0) return;
+  const int groups = (t1 - t0 + TP - 1) / TP;
+  if (groups == 0) return;
 
-  const int k0 = wave * 32 * kStreamSteps + 16 * kg;
+  const int k0 = wave * 32 * STEPS + 16 * kg;
   const __amdgpu_buffer_rsrc_t wr =
-      __builtin_amdgcn_make_buffer_rsrc((void*)a.w, (short)0, (int)(2u * (uint32_t)a.n * kStreamK), 0x00020000);
-  const int w_off = 2 * (c * kStreamK + k0);
+      __builtin_amdgcn_make_buffer_rsrc((void*)a.w, (short)0, (int)(2u * (uint32_t)a.n * kK), 0x00020000);
+  const int w_off = 2 * (c * kK + k0);
   // (past the last tile: its weights again, so that every path issues the same
   // loads and the waits count them exactly)
-  auto load_pair = [&](int p, bf16x8 (&f)[2][kStreamSteps]) {
+  auto load_group = [&](int p, bf16x8 (&f)[TP][STEPS]) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int tile_off = (int)(min(t0 + 2 * p + i, t1 - 1) * (2u * 16 * kStreamK));
+    for (int i = 0; i < TP; ++i) {
+      const int tile_off = (int)(min(t0 + TP * p + i, t1 - 1) * (2u * 16 * kK));
 #pragma unroll
-      for (int u = 0; u < kStreamSteps; ++u)
+      for (int u = 0; u < STEPS; ++u)
         f[i][u] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(wr, w_off + 2 * step_off(u), tile_off, 0));
     }
   };
-  bf16x8 f0[2][kStreamSteps], f1[2][kStreamSteps], f2[2][kStreamSteps], xf[MT][kStreamSteps];
-  load_pair(0, f0);
+  bf16x8 f0[TP][STEPS], f1[TP][STEPS], f2[TP][STEPS], xf[MT][STEPS];
+  load_group(0, f0);
 #pragma unroll
   for (int j = 0; j < MT; ++j)
 #pragma unroll
-    for (int u = 0; u < kStreamSteps; ++u)
+    for (int u = 0; u < STEPS; ++u)
       xf[j][u] = ld_op(a.x + (int64_t)min(16 * j + c, a.rows - 1) * a.x_stride + k0 + step_off(u));
-  load_pair(1, f1);
+  load_group(1, f1);
 
   const __amdgpu_buffer_rsrc_t out =
       __builtin_amdgcn_make_buffer_rsrc(a.out, (short)0, (int)(2u * (uint32_t)a.rows * (uint32_t)a.n), 0x00020000);
   const int red_tile = wave >> 2, red_m = 16 * (wave & 3) + c;
-  auto step = [&](int p, bf16x8 (&cur)[2][kStreamSteps], bf16x8 (&ahead)[2][kStreamSteps]) {
-    load_pair(p + 2, ahead);
+  auto step = [&](int p, bf16x8 (&cur)[TP][STEPS], bf16x8 (&ahead)[TP][STEPS]) {
+    load_group(p + 2, ahead);
     __builtin_amdgcn_sched_barrier(0);
-    f32x4* buf = part + (p & 1) * (kStreamWaves * 2 * MT * 64);
+    f32x4* buf = part + (p & 1) * (kStreamWaves * TP * MT * 64);
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < TP; ++i) {
       f32x4 acc[MT];
 #pragma unroll
       for (int j = 0; j < MT; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int u = 0; u < kStreamSteps; ++u)
+      for (int u = 0; u < STEPS; ++u)
 #pragma unroll
         for (int j = 0; j < MT; ++j)
           acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur[i][u], xf[j][u], acc[j], 0, 0, 0);
 #pragma unroll
-      for (int j = 0; j < MT; ++j) buf[((wave * 2 + i) * MT + j) * 64 + lane] = acc[j];
+      for (int j = 0; j < MT; ++j) buf[((wave * TP + i) * MT + j) * 64 + lane] = acc[j];
     }
     lds_barrier();
+    if (TP == 1 && red_tile) return;  // (a single tile: its rows are the first four waves')
     f32x4 sum = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int w = 0; w < kStreamWaves; ++w) {
-      const f32x4 q = buf[((w * 2 + red_tile) * MT + min(wave & 3, MT - 1)) * 64 + lane];
+      const f32x4 q = buf[((w * TP + red_tile) * MT + min(wave & 3, MT - 1)) * 64 + lane];
 #pragma unroll
       for (int r = 0; r < 4; ++r) sum[r] += q[r];
     }
     const float y[4] = {sum[0], sum[1], sum[2], sum[3]};
     const uint2 o = pack_bf16x4(y);
-    const int tile = t0 + 2 * p + red_tile;
+    const int tile = t0 + TP * p + red_tile;
     const bool ok = red_m < a.rows && tile < t1;
     const uint32_t off = ok ? 2u * ((uint32_t)red_m * (uint32_t)a.n + (uint32_t)(tile * 16 + 4 * kg)) : 0xfffffff8u;
     __builtin_amdgcn_raw_buffer_store_b64(u32x2{o.x, o.y}, out, (int)off, 0, 0);
   };
   for (int p = 0;;) {
     step(p, f0, f2);
-    if (++p >= pairs) break;
+    if (++p >= groups) break;
     step(p, f1, f0);
-    if (++p >= pairs) break;
+    if (++p >= groups) break;
     step(p, f2, f1);
-    if (++p >= pairs) break;
+    if (++p >= groups) break;
   }
 }
 
@@ -344,13 +347,25 @@ LinearPlan plan_linear(int64_t rows, int n, int k, int act, int norm) {
   if (rows < 1 || rows > kLinMaxRows || n < 16 || n % 16 || k < 32 || k % 32) return p;
   if (norm && k > kNormMaxK) return p;
   const int m_tiles = (int)(rows + 15) / 16, n_tiles = n / 16;
-  // Streaming from 8 feature tiles a CU on (its offsets are 32 bits), for more
-  // than 16 rows: at most 16 are as fast or faster in the library (151936 x
-  // 1024: one row 62 us and 63 here, 16 rows 65 and 69, 17 rows 75 and 70).
+  // Streaming, for more than 16 rows (at most 16 are as fast or faster in the
+  // library: 151936 x 1024 one row 62 us and 63 here, 16 rows 65 / 69), of k up
+  // to what a wave holds of x and offsets of 32 bits, from 16 feature tiles a CU
+  // on (8 at k 512): with fewer, a range's whole groups weigh too much (40 rows,
+  // 50272 features: k 1024 22.4 us and 27.3 here, 1536 33.6 / 35.8).  From there
+  // on the library goes from a little faster to half as fast, with its own
+  // tiling: 40 rows, k 512 / 1024 / 1536 / 2048: 79984 features 42.2 / 58.7 / 83.0
+  // / 80.1 and 20.3 / 39.3 / 54.6 / 72.7 here, 115200 32.1 / 52.7 / 86.1 / 102.9
+  // and 28.3 / 56.1 / 76.7 / 101.7, 128256 41.1 / 57.3 / 101.4 / 123.6 and 31.2 /
+  // 59.1 / 86.3 / 110.0, 200064 102.4 / 144.0 / 200.9 / 195.1 and 47.0 / 90.4 /
+  // 134.7 / 167.3, 256000 61.7 / 111.8 / 171.5 / 233.7 and 58.7 / 114.2 / 168.8 /
+  // 212.4.
   if (!act && n_tiles >= 8 * kCus) {
-    if (norm || k != kStreamK || m_tiles < 2 || (int64_t)k * n * 2 >= ((int64_t)1 << 31)) return p;
+    if (norm || k % 512 || k > 2048 || m_tiles < 2 || n_tiles < (k == 512 ? 8 : 16) * kCus ||
+        (int64_t)k * n * 2 >= ((int64_t)1 << 31))
+      return p;
     p.kind = 2;
     p.mt = m_tiles;
+    p.blk = k / 256;
     return p;
   }
   // Split up to 2^20 (feature tiles x row tiles x k: 32 MB of x read by the
@@ -413,10 +428,15 @@ void launch_rows(const LinearArgs& a, const LinearPlan& p, hipStream_t s) {
   else launch_split<1, ACT, NORM>(a, p, s);
 }
 
-template <int MT>
-void launch_stream(const LinearArgs& a, hipStream_t s) {
-  const size_t lds = (size_t)2 * kStreamWaves * 2 * MT * 64 * sizeof(f32x4);
-  hipLaunchKernelGGL(linear_stream_kernel<MT>, dim3(kCus), dim3(kStreamWaves * kWave), lds, s, a);
+template <int STEPS>
+void launch_stream(const LinearArgs& a, int mt, hipStream_t s) {
+  const dim3 grid(kCus), block(kStreamWaves * kWave);
+  const size_t lds = (size_t)2 * kStreamWaves * (STEPS <= 4 ? 2 : 1) * mt * 64 * sizeof(f32x4);
+  switch (mt) {
+    case 2: hipLaunchKernelGGL((linear_stream_kernel<2, STEPS>), grid, block, lds, s, a); break;
+    case 3: hipLaunchKernelGGL((linear_stream_kernel<3, STEPS>), grid, block, lds, s, a); break;
+    default: hipLaunchKernelGGL((linear_stream_kernel<4, STEPS>), grid, block, lds, s, a); break;
+  }
 }
 
 }  // namespace
@@ -446,10 +466,11 @@ extern "C" int mkv_linear(void* out, const void* x, int64_t x_row_stride, const 
                reinterpret_cast<const uint16_t*>(norm_weight), eps, reinterpret_cast<const uint16_t*>(residual)};
   const int m_tiles = (int)(rows + 15) / 16;
   if (p.kind == 2) {
-    switch (p.mt) {
-      case 2: launch_stream<2>(a, s); break;
-      case 3: launch_stream<3>(a, s); break;
-      default: launch_stream<4>(a, s); break;
+    switch (p.blk) {
+      case 2: launch_stream<2>(a, p.mt, s); break;
+      case 4: launch_stream<4>(a, p.mt, s); break;
+      case 6: launch_stream<6>(a, p.mt, s); break;
+      default: launch_stream<8>(a, p.mt, s); break;
     }
   } else {
     a.m_groups = (m_tiles + p.mt - 1) / p.mt;

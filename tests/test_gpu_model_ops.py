@@ -77,7 +77,7 @@ def _ulp(x):
 
 
 @pytest.mark.parametrize("rows", [1, 15, 16, 17, 33, 60, 64])
-@pytest.mark.parametrize("n,k", [(16, 512), (48, 768), (4096, 1024), (1024, 2048), (112, 3072), (80, 4096), (48, 1536), (32816, 1024)])
+@pytest.mark.parametrize("n,k", [(16, 512), (48, 768), (4096, 1024), (1024, 2048), (112, 3072), (80, 4096), (48, 1536), (65584, 1024)])
 @pytest.mark.parametrize("strided", [False, True])
 def test_linear(dev, rows, n, k, strided):
     """mkv_linear in every form (4, 8 and 16 waves, 4 and 6 k-steps, one or
@@ -199,6 +199,14 @@ def test_model_layers_with_and_without_fused_products(dev, monkeypatch):
     err = float((got - want).norm() / want.norm())
     print("relative difference", err)
     assert err < 6 * 2.0 ** -8
+
+
+@pytest.mark.parametrize("rows", [17, 40, 60])
+@pytest.mark.parametrize("n,k", [(32816, 512), (65552, 1536), (65568, 2048)])
+def test_linear_streaming_widths(dev, rows, n, k):
+    """The streaming form's other widths (2, 6 and 8 k-steps a wave, pairs of
+    feature tiles and single ones), with ranges of tiles that differ by one."""
+    test_linear(dev, rows, n, k, rows % 2 == 1)
 
 
 # Sizes in the forms that the tests above leave out: k in 4, 8 and 16 parts of

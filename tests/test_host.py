@@ -279,6 +279,25 @@ def test_products_leave_a_second_round_to_the_library():
     assert taken(32, 3072, 2048) and taken(16, 24576, 512) and taken(16, 8192, 2048, 0, 1)
 
 
+def test_streaming_products_by_size():
+    """The streaming form of mkv_linear (LM heads): k of 512 to 2048 in steps
+    of 512, more than 16 rows, 16 feature tiles a CU (8 at k 512), weights of
+    less than 2 GiB, no norm."""
+    lib = _lib.load()
+
+    def taken(rows, n, k, norm=0):
+        return lib.mkv_linear_supported(rows, n, k, 0, norm, _lib.DTYPE_BF16)
+
+    for k in (512, 1024, 1536, 2048):
+        first = 32768 if k == 512 else 65536
+        assert taken(17, first, k) and taken(64, 262144, k) and not taken(16, 262144, k)
+        assert not taken(17, first, k, 1) and not taken(65, first, k)
+        assert k == 512 or not (taken(17, first - 16, k) or taken(64, 32768, k))
+        most = (2 ** 30 - 1) // k // 16 * 16
+        assert taken(64, most, k) and not taken(64, most + 16, k)
+    assert not any(taken(32, 131072, k) for k in (256, 768, 1280, 2560, 4096))
+
+
 def test_decode_route_choice():
     """The library's schedule for split_tokens 0 (mkv_paged_decode_route on
     a 256-CU device), for the decode workloads that are measured, and the
