@@ -36,6 +36,8 @@ from dataclasses import dataclass, field
 import torch
 import torch.nn.functional as F
 from torch.autograd import forward_ad
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from . import _lib
 from . import context as C
@@ -273,11 +275,15 @@ def _own_weight(w: torch.Tensor, rows: int, n: int, act: int, norm: int = 0) -> 
 def _plain(*tensors: torch.Tensor) -> bool:
     """Whether a kernel on the tensors' memory is all that a product of them
     means: nothing traces or intercepts it (torch.compile, jit, dispatch
-    modes), and no tensor is a subclass's, one of a function transform's
-    (vmap, jvp) or carries a forward-mode tangent."""
+    modes, function modes other than a default device), autocast leaves bf16
+    alone, and no tensor is a subclass's, sparse, one of a function
+    transform's (vmap, jvp) or carries a forward-mode tangent."""
     return (not torch.compiler.is_compiling() and not torch.jit.is_tracing()
             and torch._C._len_torch_dispatch_stack() == 0
-            and all(type(t) in (torch.Tensor, torch.nn.Parameter)
+            and (torch._C._len_torch_function_stack() == 0
+                 or all(type(m) is DeviceContext for m in _get_current_function_mode_stack()))
+            and not (torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != torch.bfloat16)
+            and all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.layout is torch.strided
                     and not torch._C._functorch.is_functorch_wrapped_tensor(t)
                     and forward_ad.unpack_dual(t).tangent is None for t in tensors))
 

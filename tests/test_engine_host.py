@@ -10,6 +10,7 @@ import random
 
 import pytest
 import torch
+import torch.overrides
 
 from mkv import engine as E
 
@@ -171,3 +172,32 @@ def test_products_under_transforms_are_left_to_torch():
     w = w.detach()
     assert torch.allclose(torch.jit.trace(f, x, check_trace=False)(2 * x), 2 * want)
     assert len(seen) == 7 and not any(seen)
+
+
+def test_products_under_modes_and_autocast_are_left_to_torch():
+    """A function mode sees the engine's products (a default device is none of
+    their business), autocast to another type rounds them to it, and a sparse
+    weight is torch's to multiply."""
+    class Seen(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            calls.append(func)
+            return func(*args, **(kwargs or {}))
+
+    calls = []
+    x, w = torch.randn(3, 8), torch.randn(4, 8)
+    with Seen():
+        plain = E._plain(x, w)
+        E.linear(x, w)
+    assert not plain and torch.nn.functional.linear in calls
+    with torch.device("cpu"):
+        assert E._plain(x, w)
+    was = torch.get_autocast_dtype("cuda")
+    torch.set_autocast_enabled("cuda", True)  # (torch.autocast wants a GPU for it)
+    try:
+        for dtype in (torch.bfloat16, torch.float16):
+            torch.set_autocast_dtype("cuda", dtype)
+            assert E._plain(x, w) == (dtype is torch.bfloat16)
+    finally:
+        torch.set_autocast_enabled("cuda", False)
+        torch.set_autocast_dtype("cuda", was)
+    assert not E._plain(x, w.to_sparse_csr()) and E._plain(x, w)
