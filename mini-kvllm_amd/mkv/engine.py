@@ -29,6 +29,7 @@ tokens per second; it is not a port of the reference's runner.  The pieces:
 """
 from __future__ import annotations
 
+import functools
 import time
 from collections import deque
 from dataclasses import dataclass, field
@@ -44,6 +45,12 @@ from . import context as C
 from .attention import DECODE_STREAM, DECODE_WORKGROUP, Attention, _dtype_code, _stream
 from .decode_state import DecodeGraphs, DecodeMetadata
 from .producer import qkv_norm_rope_append, qkv_norm_rope_append_decode
+
+_is_tracing = torch._C._is_tracing
+_dispatch_modes = torch._C._len_torch_dispatch_stack
+_function_modes = torch._C._len_torch_function_stack
+_is_transformed = torch._C._functorch.is_functorch_wrapped_tensor
+_PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
 
 
 # ---------------------------------------------------------------------------
@@ -264,52 +271,74 @@ def silu_and_mul(x: torch.Tensor) -> torch.Tensor:
     return out
 
 
+@functools.lru_cache(maxsize=1024)
+def _own_size(rows: int, n: int, k: int, act: int, norm: int) -> bool:
+    """Whether mkv_linear takes a bf16 product of these sizes."""
+    return bool(_lib.query("mkv_linear_supported", rows, n, k, act, norm, _lib.DTYPE_BF16))
+
+
+# An eager decode step's host time is mostly what surrounds its launches.  60
+# sequences through 28 layers, 113 products, keep the GPU busy for 1.65 ms; with
+# a library query and unpack_dual for every product the host took 1.84.
 def _own_weight(w: torch.Tensor, rows: int, n: int, act: int, norm: int = 0) -> bool:
     """Whether mkv_linear takes the product of this many rows with w: bf16 on
     the GPU, no gradient to record, in sizes it shares out evenly."""
-    return (w.is_cuda and w.dtype == torch.bfloat16 and w.dim() == 2 and w.shape[0] == (1 + act) * n
-            and w.is_contiguous() and w.data_ptr() % 16 == 0 and not (torch.is_grad_enabled() and w.requires_grad)
-            and bool(_lib.query("mkv_linear_supported", rows, n, w.shape[1], act, norm, _lib.DTYPE_BF16)))
+    shape = w.shape
+    return (w.is_cuda and w.dtype is torch.bfloat16 and len(shape) == 2 and shape[0] == (1 + act) * n
+            and w.is_contiguous() and w.data_ptr() % 16 == 0 and not (w.requires_grad and torch.is_grad_enabled())
+            and _own_size(rows, n, shape[1], act, norm))
 
 
-def _plain(*tensors: torch.Tensor) -> bool:
+def _untouched() -> bool:
+    """Whether nothing traces or intercepts what torch does (torch.compile,
+    jit, dispatch modes, function modes other than a default device) and
+    autocast leaves bf16 alone."""
+    return not (torch.compiler.is_compiling() or _is_tracing() or _dispatch_modes()
+                or (_function_modes()
+                    and any(type(m) is not DeviceContext for m in _get_current_function_mode_stack()))
+                or (torch.is_autocast_enabled() and torch.get_autocast_dtype("cuda") != torch.bfloat16))
+
+
+def _plain(*tensors: torch.Tensor, untouched: bool | None = None) -> bool:
     """Whether a kernel on the tensors' memory is all that a product of them
-    means: nothing traces or intercepts it (torch.compile, jit, dispatch
-    modes, function modes other than a default device), autocast leaves bf16
-    alone, and no tensor is a subclass's, sparse, one of a function
-    transform's (vmap, jvp) or carries a forward-mode tangent."""
-    return (not torch.compiler.is_compiling() and not torch.jit.is_tracing()
-            and torch._C._len_torch_dispatch_stack() == 0
-            and (torch._C._len_torch_function_stack() == 0
-                 or all(type(m) is DeviceContext for m in _get_current_function_mode_stack()))
-            and not (torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != torch.bfloat16)
-            and all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.layout is torch.strided
-                    and not torch._C._functorch.is_functorch_wrapped_tensor(t)
-                    and forward_ad.unpack_dual(t).tangent is None for t in tensors))
+    means: _untouched (None: asked for here), and no tensor is a subclass's,
+    sparse, one of a function transform's (vmap, jvp) or carries a
+    forward-mode tangent (none does outside a dual level)."""
+    if not (_untouched() if untouched is None else untouched):
+        return False
+    for t in tensors:
+        if (type(t) not in _PLAIN_TYPES or t.layout is not torch.strided or _is_transformed(t)
+                or (forward_ad._current_level >= 0 and forward_ad.unpack_dual(t).tangent is not None)):
+            return False
+    return True
 
 
 def _own_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether mkv_linear reads x's rows as they are, for a w it takes (on the
     current device: it launches there)."""
-    return (x.device == w.device and x.get_device() == torch.cuda.current_device() and x.dtype == w.dtype and x.dim() == 2 and x.shape[1] == w.shape[1]
-            and x.stride(1) == 1 and x.shape[1] <= x.stride(0) <= 1 << 20 and x.stride(0) % 8 == 0
-            and x.data_ptr() % 16 == 0 and not (torch.is_grad_enabled() and x.requires_grad))
+    shape, k = x.shape, w.shape[1]
+    if len(shape) != 2 or shape[1] != k or x.dtype is not w.dtype:
+        return False
+    s0, s1 = x.stride()
+    return (s1 == 1 and k <= s0 <= 1 << 20 and s0 % 8 == 0 and x.data_ptr() % 16 == 0
+            and x.get_device() == w.get_device() == torch.cuda.current_device()
+            and not (x.requires_grad and torch.is_grad_enabled()))
 
 
-def _own_product(x: torch.Tensor, w: torch.Tensor, n: int, act: int, norm: int = 0) -> bool:
-    return (_plain(x, w) and x.dim() == 2 and 0 < x.shape[0] <= 64
-            and _own_weight(w, x.shape[0], n, act, norm) and _own_rows(x, w))
+def _own_product(x: torch.Tensor, w: torch.Tensor, n: int, act: int, norm: int = 0,
+                 untouched: bool | None = None) -> bool:
+    return (_plain(x, w, untouched=untouched) and x.dim() == 2 and 0 < (rows := x.shape[0]) <= 64
+            and _own_weight(w, rows, n, act, norm) and _own_rows(x, w))
 
 
 def _product(x: torch.Tensor, w: torch.Tensor, n: int, act: int = 0, norm: torch.Tensor | None = None,
              eps: float = 0.0, residual: torch.Tensor | None = None) -> torch.Tensor:
-    out = residual
-    if out is None:
-        out = torch.empty(x.shape[0], n, dtype=x.dtype, device=x.device)
-    _lib.call("mkv_linear", out.data_ptr(), x.data_ptr(), x.stride(0), w.data_ptr(),
-              norm.data_ptr() if norm is not None else None, float(eps),
-              residual.data_ptr() if residual is not None else None, x.shape[0], n,
-              x.shape[1], act, _dtype_code(x, "x"), _stream(x.device))
+    rows, k = x.shape
+    out = residual if residual is not None else x.new_empty(rows, n)
+    out_ptr = out.data_ptr()
+    _lib.call("mkv_linear", out_ptr, x.data_ptr(), x.stride(0), w.data_ptr(),
+              norm.data_ptr() if norm is not None else None, eps, out_ptr if residual is not None else None,
+              rows, n, k, act, _lib.DTYPE_BF16, _stream(x.device))
     return out
 
 
@@ -327,28 +356,32 @@ def gated_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 
 def normed_linear(x: torch.Tensor | None, residual: torch.Tensor, norm: torch.Tensor, eps: float,
-                  w: torch.Tensor, act: int = 0) -> torch.Tensor:
+                  w: torch.Tensor, act: int = 0, untouched: bool | None = None) -> torch.Tensor:
     """The (gated, with act) product of the RMS-normalised residual stream:
     residual, plus x where that is not None (the sum is then left in
     residual).  With nothing to add the norm runs inside the product where
-    mkv_linear takes it, else the add and the norm are a kernel ahead of it."""
+    mkv_linear takes it, else the add and the norm are a kernel ahead of it.
+    untouched: _untouched(), for a caller with many products."""
     n = w.shape[0] // (1 + act)
-    if (x is None and norm.device == w.device and norm.dtype == w.dtype and norm.shape == w.shape[1:]
-            and norm.is_contiguous() and norm.data_ptr() % 16 == 0 and _own_product(residual, w, n, act, 1)):
+    if (x is None and _own_product(residual, w, n, act, 1, untouched) and norm.dtype is w.dtype
+            and norm.dim() == 1 and norm.numel() == w.shape[1] and norm.is_contiguous()
+            and norm.get_device() == w.get_device() and norm.data_ptr() % 16 == 0):
         return _product(residual, w, n, act, norm, eps)
     h = rms_norm(residual, norm, eps) if x is None else rms_norm(x, norm, eps, residual)
     return gated_linear(h, w) if act else linear(h, w)
 
 
-def add_linear(residual: torch.Tensor, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor | None:
+def add_linear(residual: torch.Tensor, x: torch.Tensor, w: torch.Tensor,
+               untouched: bool | None = None) -> torch.Tensor | None:
     """residual += x w^T in the product's epilogue (None) where mkv_linear
     takes the rows and the weight as they are, else the product, which is then
     still to be added."""
-    if (residual.shape == (*x.shape[:-1], w.shape[0]) and residual.is_contiguous() and residual.dtype == w.dtype
-            and residual.device == w.device and residual.data_ptr() % 16 == 0
-            and w.shape[0] < 32768  # (more features take no residual)
-            and _own_product(x, w, w.shape[0], 0)):
-        _product(x, w, w.shape[0], residual=residual)
+    n = w.shape[0]
+    if (n < 32768  # (more features take no residual)
+            and _own_product(x, w, n, 0, 0, untouched) and residual.shape == (x.shape[0], n)
+            and residual.is_contiguous() and residual.dtype is w.dtype
+            and residual.get_device() == w.get_device() and residual.data_ptr() % 16 == 0):
+        _product(x, w, n, residual=residual)
         return None
     return linear(x, w)
 
@@ -449,8 +482,9 @@ class Qwen3Model(torch.nn.Module):
         # products that mkv_linear takes the norms and residual additions are
         # part of them (five launches a layer instead of seven).
         x, residual = None, F.embedding(input_ids, self.embed)
+        free = _untouched()
         for li, lay in enumerate(self.layers):
-            qkv = normed_linear(x, residual, lay["in_norm"], cfg.eps, lay["qkv"])
+            qkv = normed_linear(x, residual, lay["in_norm"], cfg.eps, lay["qkv"], 0, free)
             att = lay["attn"]
             ctx = C.current_context()
             if self.fuse_decode_step and not ctx.is_prefill:
@@ -469,9 +503,9 @@ class Qwen3Model(torch.nn.Module):
                     eps=cfg.eps, kv_cache_dtype=att.kv_cache_dtype, k_scale=att.k_scale,
                     v_scale=att.v_scale, return_k=full_prefill)
                 o = self.attention(li, q, k, v)
-            x = add_linear(residual, o, lay["o"])
-            h = normed_linear(x, residual, lay["post_norm"], cfg.eps, lay["gate_up"], 1)
-            x = add_linear(residual, h, lay["down"])
+            x = add_linear(residual, o, lay["o"], free)
+            h = normed_linear(x, residual, lay["post_norm"], cfg.eps, lay["gate_up"], 1, free)
+            x = add_linear(residual, h, lay["down"], free)
         if x is None:
             return rms_norm(residual, self.final_norm, cfg.eps)
         return rms_norm(x, self.final_norm, cfg.eps, residual)

@@ -201,3 +201,20 @@ def test_products_under_modes_and_autocast_are_left_to_torch():
         torch.set_autocast_enabled("cuda", False)
         torch.set_autocast_dtype("cuda", was)
     assert not E._plain(x, w.to_sparse_csr()) and E._plain(x, w)
+
+
+def test_products_ask_little_of_the_host(monkeypatch):
+    """A product's checks query the library once for each set of sizes and
+    unpack no tensor outside a dual level: with both for every product an
+    eager decode step was paced by the host."""
+    from torch.autograd import forward_ad
+
+    calls = []
+    query, unpack = E._lib.query, forward_ad.unpack_dual
+    monkeypatch.setattr(E._lib, "query", lambda *a: (calls.append(a[0]), query(*a))[1])
+    monkeypatch.setattr(forward_ad, "unpack_dual", lambda *a: (calls.append("unpack_dual"), unpack(*a))[1])
+    E._own_size.cache_clear()
+    x, w = torch.randn(3, 8), torch.randn(4, 8)
+    for _ in range(3):
+        assert E._plain(x, w) and E._own_size(60, 4096, 1024, 0, 1) and not E._own_size(65, 4096, 1024, 0, 1)
+    assert calls == ["mkv_linear_supported"] * 2
