@@ -216,10 +216,11 @@ int mkv_fp8_calibrate_per_tensor(const void* key, int64_t key_row_stride,
  *       widest context the table allows gives each of its waves at most 128
  *       tokens, or at most 256 tokens when its waves also fill enough of
  *       the device (per-tensor FP8: 2 x CUs waves, BF16/F16: 6 x CUs;
- *       never for per-token-head scales; FP32: at most 512 tokens and
- *       2 x CUs waves); else stream-K (BF16/F16/FP8/INT8 KV, batch <= 8192),
- *       else split-K with a library-chosen split (mkv_paged_decode_route
- *       reports the choice);
+ *       never for per-token-head scales) (FP32 instead: 2 x CUs waves of
+ *       at most 64 tokens, or of at most 512 where the table holds at most
+ *       1024 and every CU has a (sequence, KV head) pair); else stream-K
+ *       (BF16/F16/FP8/INT8 KV, batch <= 8192), else split-K with a
+ *       library-chosen split (mkv_paged_decode_route reports the choice);
  *   MKV_DECODE_STREAM = stream-K over 32-token tiles on a persistent grid,
  *       groups of num_kv_heads waves sharing each tile range, and a merge
  *       kernel (split-K where stream-K does not apply);

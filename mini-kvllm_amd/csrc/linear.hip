@@ -13,9 +13,13 @@
 // waves of a workgroup until a wave's share is one memory round trip, and
 // there are about as many workgroups as CUs.  60 rows, weights not in cache,
 // us a product, before (the library's products, the gated one with
-// mkv_silu_mul behind it) and now: 4096 x 1024 11.3 / 6.2, 1024 x 2048 8.0 /
-// 5.2, 1024 x 3072 12.0 / 7.4, 2 x 3072 x 1024 gated 14.7 / 9.3, 151936 x 1024
-// 83 / 78; one row: 7.5 / 4.4, 8.4 / 4.9, 11.8 / 6.4, 10.4 / 5.6.
+// mkv_silu_mul behind it) and now: 4096 x 1024 11.2 / 6.3, 1024 x 2048 9.7 /
+// 5.3, 1024 x 3072 12.0 / 7.5, 2 x 3072 x 1024 gated 14.7 / 9.3, 151936 x 1024
+// 85 / 76; one row: 7.5 / 4.5, 8.7 / 5.0, 11.9 / 6.6, 10.4 / 5.6.  With the
+// residual added 1024 x 2048 takes 5.4 and 1024 x 3072 7.7; normalised (before:
+// behind mkv_rmsnorm with its residual addition) 4096 x 1024 15.1 / 9.6 and the
+// gated one 18.5 / 11.2, one row 10.8 / 5.4 and 13.7 / 6.8: those are the forms
+// of a decoder layer.
 //
 // The MFMA's rows are 16 output features (A = W, straight from memory: the
 // loads of two k-steps cover 16 whole lines), its columns 16 rows of x, so a
